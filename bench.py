@@ -105,14 +105,16 @@ def live_columns(n: int, d: float) -> int:
     return int(np.count_nonzero(fy * fy <= filt * filt))
 
 
-def compulsory_bytes(name: str, ctx) -> float:
-    """HBM bytes one launch of `name` must move in this workload (mean over
-    its launches), at the data types the kernels use.
+def compulsory_bytes(name: str, ctx, launches: float) -> float:
+    """HBM bytes one launch of `name` (launched `launches` times per step) must
+    move in this workload (mean over its launches), at the data types the
+    kernels use.
 
     With B molecules, n x n waves, H = n/2 + 1 half-spectrum columns, nE
     elements, nS slices and L live wave columns:
-      k_spec_sparse          Y write B n H 8 + form factors nE n H 4
-                             + row table B nE n 4 + atom y bins 2 per binned atom
+      k_spec_sparse          (a launch takes nS / launches slices) per slice Y write
+                             B n H 8 + row table B nE n 4 + atom y bins 2 per binned
+                             atom; per launch form factors nE n H 4
       k_slice_pass_a         Y read B n H 8 + wave write B n L 8
                              + wave read B n L 8 (not on the first slice)
       k_col_fft_mul_ifft     wave read + write B n L 16 (last slice: all n columns)
@@ -132,8 +134,8 @@ def compulsory_bytes(name: str, ctx) -> float:
     npix = n * n
     atoms = ctx["n_atoms"]
     per = {
-        "k_spec_sparse": B * n * H * 8.0 + nE * n * H * 4.0 + B * nE * n * 4.0
-        + 2.0 * ctx["binned_atoms"] / nS,
+        "k_spec_sparse": (nS * (B * n * H * 8.0 + B * nE * n * 4.0) + 2.0 * ctx["binned_atoms"])
+        / launches + nE * n * H * 4.0,
         "k_slice_pass_a": B * n * H * 8.0 + B * n * L * 8.0 + B * n * L * 8.0 * (nS - 1) / nS,
         "k_col_fft_mul_ifft": B * n * 16.0 * (L * (nS - 1) + n) / nS,
         "k_row_ifft_intensity": 12.0 * npix * B,
@@ -710,7 +712,7 @@ def main():
     step_measured = 0.0
     step_measured_ok = traffic is not None and bool(kernels)
     for k in sorted(kernels, key=lambda r: -r["total_ms"]):
-        b = compulsory_bytes(k["name"], ctx)
+        b = compulsory_bytes(k["name"], ctx, k["count"] / args.steps)
         mean_s = k["mean_ms"] * 1e-3
         row = {"kernel": k["name"], "launches_per_step": k["count"] / args.steps,
                "mean_us": round(k["mean_ms"] * 1e3, 2),

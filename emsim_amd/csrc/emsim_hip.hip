@@ -430,6 +430,9 @@ int launch_row_ifft_intensity(const float2* in, float* out, int64_t rows, const 
 struct ColDead {
     int lo = 1 << 30, hi = -1;
     bool skip_tiles = false;
+    // the mean's rounding rests, one per image, or null; first: none yet
+    float2* carry = nullptr;
+    bool carry_first = true;
 };
 
 template <int N, class Mul, int SHAPE = 0>
@@ -478,7 +481,7 @@ int launch_col_mul_shape(float2* data, int ld, int ncols, int64_t img_stride, in
     const RunSched sched{(int)(strips / pairs), (int)(strips % pairs)};
     const dim3 grid((unsigned)(2 * pairs));
     EMSIM_LAUNCH(N, (k_col_fft_mul_ifft<N, Mul, SHAPE>), grid, dim3(Cfg::BLOCK), 0, s, data, ld,
-                 ncols, dc, img_stride, n_tiles, sched, mul, tw);
+                 ncols, dc, img_stride, n_tiles, sched, mul, cd.carry, cd.carry_first, tw);
     return EMSIM_HIP_OK;
 }
 
@@ -1449,19 +1452,22 @@ namespace {
 
 template <int N>
 int launch_spec_sparse(const uint32_t* row_start, const uint16_t* bucket, const float* sf,
-                       const float* sft, float2* Y, int slice, int n_slices, int n_elems, int H,
-                       int ldh, int n2, int bandlimit, int band_r2, float inv_npix, int batch,
-                       const int* order, const float2* tw, hipStream_t s) {
+                       const float* sft, float2* Y, int slice0, int n_sc, int n_slices,
+                       int n_elems, int H, int ldh, int n2, int bandlimit, int band_r2,
+                       float inv_npix, int batch, const int* order, const float2* tw,
+                       hipStream_t s) {
     using Cfg = SpecCfg<N>;
     if (H != n2 / 2 + 1 || n2 < 2 || ldh < H + n_elems)
         return fail(EMSIM_HIP_EINVAL, "spectrum: needs H = n2/2 + 1, n2 >= 2, ldh >= H + n_elems");
     // with spec_pack(N), column n2/2 is carried by column 0
     const int cols = spec_pack(N) ? n2 / 2 : H;
-    const dim3 grid((unsigned)(ceil_div(cols, Cfg::C) * (int64_t)batch));
+    const int64_t blocks = ceil_div(cols, Cfg::C) * (int64_t)batch * n_sc;
+    if (blocks >= ((int64_t)1 << 31))
+        return fail(EMSIM_HIP_EINVAL, "spectrum: %lld blocks, at most 2^31 - 1", (long long)blocks);
     if (!sft) return fail(EMSIM_HIP_EINVAL, "spectrum: no tile-major form-factor table");
-    EMSIM_LAUNCH(N, (k_spec_sparse<N>), grid, dim3(Cfg::BLOCK), 0, s, row_start, bucket, sf,
-                 sft, Y, slice, n_slices, n_elems, H, ldh, n2, batch, bandlimit, band_r2,
-                 inv_npix, order, tw);
+    EMSIM_LAUNCH(N, (k_spec_sparse<N>), dim3((unsigned)blocks), dim3(Cfg::BLOCK), 0, s, row_start,
+                 bucket, sf, sft, Y, slice0, n_sc, n_slices, n_elems, H, ldh, n2, batch, bandlimit,
+                 band_r2, inv_npix, order, tw);
     return EMSIM_HIP_OK;
 }
 
@@ -1501,6 +1507,42 @@ int launch_slice_pass_a(bool first, const float2* Y, float2* wave, int64_t n_pai
     return EMSIM_HIP_OK;
 }
 
+// The transmission functions of n_sc slices, and one slice's wave rows through
+// them (pass A in two kernels).
+template <int N>
+int launch_phase_rows(const float2* Y, float2* phase, int n_sc, int batch, int n1, int ldh,
+                      float factor, float* vout, int slice0, int n_slices, const float2* tw,
+                      hipStream_t s) {
+    static int resident_cache[64];
+    const int64_t n_pairs = (int64_t)n_sc * batch * (n1 / 2), plane = (int64_t)n1 * N;
+    int rpw;
+    dim3 grid;
+    row_grid<N>(n_pairs, rpw, grid,
+                resident_blocks(k_phase_rows<N>, RowCfg<N>::BLOCK, resident_cache));
+    EMSIM_LAUNCH(N, (k_phase_rows<N>), grid, dim3(RowCfg<N>::BLOCK), 0, s,
+                 (OpPhaseRows<N>{Y, phase, ldh, factor, vout, n_slices * plane, slice0 * plane, n1,
+                                 batch}),
+                 n_pairs, rpw, tw);
+    return EMSIM_HIP_OK;
+}
+template <int N>
+int launch_phase_apply(bool first, const float2* phase, float2* wave, int64_t rows, float psi0,
+                       ColDead cd, const float2* tw, hipStream_t s) {
+    static int resident_cache[64];
+    int rpw;
+    dim3 grid;
+    row_grid<N>(rows, rpw, grid,
+                resident_blocks(k_phase_apply<N, false>, RowCfg<N>::BLOCK, resident_cache));
+    const dim3 block(RowCfg<N>::BLOCK);
+    if (first)
+        EMSIM_LAUNCH(N, (k_phase_apply<N, true>), grid, block, 0, s,
+                     (OpPhaseApply<N, true>{phase, wave, psi0, cd.lo, cd.hi}), rows, rpw, tw);
+    else
+        EMSIM_LAUNCH(N, (k_phase_apply<N, false>), grid, block, 0, s,
+                     (OpPhaseApply<N, false>{phase, wave, psi0, cd.lo, cd.hi}), rows, rpw, tw);
+    return EMSIM_HIP_OK;
+}
+
 template <int N>
 int launch_col_lensprop(float2* data, int ld, int ncols, int64_t img_stride, int n_img,
                         LensPropMul mul, const float2* tw, hipStream_t s, ColDead cd) {
@@ -1508,11 +1550,21 @@ int launch_col_lensprop(float2* data, int ld, int ncols, int64_t img_stride, int
 }
 
 int spec_sparse(int n, const uint32_t* row_start, const uint16_t* bucket, const float* sf,
-                const float* sft, float2* Y, int slice, int n_slices, int n_elems, int H, int ldh,
-                int n2, int bandlimit, int band_r2, float inv_npix, int batch, const int* order,
-                const float2* tw, hipStream_t s) {
-    EMSIM_DISPATCH(n, launch_spec_sparse, row_start, bucket, sf, sft, Y, slice, n_slices,
+                const float* sft, float2* Y, int slice0, int n_sc, int n_slices, int n_elems,
+                int H, int ldh, int n2, int bandlimit, int band_r2, float inv_npix, int batch,
+                const int* order, const float2* tw, hipStream_t s) {
+    EMSIM_DISPATCH(n, launch_spec_sparse, row_start, bucket, sf, sft, Y, slice0, n_sc, n_slices,
                    n_elems, H, ldh, n2, bandlimit, band_r2, inv_npix, batch, order, tw, s);
+}
+int phase_rows(int n, const float2* Y, float2* phase, int n_sc, int batch, int n1, int ldh,
+               float factor, float* vout, int slice0, int n_slices, const float2* tw,
+               hipStream_t s) {
+    EMSIM_DISPATCH(n, launch_phase_rows, Y, phase, n_sc, batch, n1, ldh, factor, vout, slice0,
+                   n_slices, tw, s);
+}
+int phase_apply(int n, bool first, const float2* phase, float2* wave, int64_t rows, float psi0,
+                ColDead cd, const float2* tw, hipStream_t s) {
+    EMSIM_DISPATCH(n, launch_phase_apply, first, phase, wave, rows, psi0, cd, tw, s);
 }
 int slice_pass_a(int n, bool first, const float2* Y, float2* wave, int64_t n_pairs, int ldh,
                  float psi0, float factor, float* vout, int slice, int n_slices, int n1,
@@ -1525,7 +1577,41 @@ int col_lensprop(int n, float2* data, int ld, int ncols, int64_t img_stride, int
     EMSIM_DISPATCH(n, launch_col_lensprop, data, ld, ncols, img_stride, n_img, mul, tw, s, cd);
 }
 
+// Pass A in two kernels (transmission functions of a chunk of slices, then
+// per slice only the wave's transforms) for batches of at most this many
+// pixels: below it the per-slice pass is one short round of waves and its
+// chain of dependent transforms is the time (one 256^2 image of 45 slices
+// 740 -> 580 us, eight 128^2 images of 50 slices 797 -> 625 us, two 512^2
+// images 1,083 -> 1,020 us); above it the extra traffic costs more than the
+// shorter chain saves (four 512^2 images 1,433 -> 1,500 us, 64 of 256^2
+// 3,440 -> 4,190 us).
+constexpr int64_t kSplitPixels = (int64_t)2 * 512 * 512;
+bool fused_split(const emsim_hip_slice_builder* b, int batch) {
+    return (int64_t)batch * b->n1 * b->n2 <= kSplitPixels;
+}
+// Slices whose half spectra (and, split, transmission functions) one launch
+// builds.  The spectrum pass does not depend on the wave, so a small batch
+// takes as many slices at once as fit kChunkBytes of planes -- most of the
+// 256 MB cache behind the L2s, from which they are read back -- instead of
+// one part-filled round of blocks per slice (one 256^2 image, 45 slices:
+// 1,526 -> 740 us; 64 of 256^2 4,124 -> 3,440 us).  Large batches still take
+// kMinChunk: their planes spill to HBM, but one launch of many rounds has one
+// tail instead of one per slice (64 of 512^2 x 100: 18.53 ms at one slice,
+// 18.12 ms at seven; 64 / 128 / 192 / 256 MB with no minimum measured 6,145 /
+// 5,478 / 5,352 / 5,424 us for 32 of 512^2 x 50).
+constexpr int64_t kChunkBytes = (int64_t)192 << 20;
+constexpr int64_t kMinChunk = 8;
+int fused_chunk(const emsim_hip_slice_builder* b, int batch) {
+    const int64_t rows = (int64_t)batch * b->n1;
+    const int64_t per = rows * (fused_ld(b) + (fused_split(b, batch) ? b->n2 : 0)) *
+                        (int64_t)sizeof(float2);
+    const int64_t c = std::max(kChunkBytes / per, kMinChunk);
+    return (int)std::min(c, (int64_t)b->n_slices);
+}
+
 struct FusedWorkspace {
+    int chunk;        // slices per launch of the spectrum pass
+    float2* phase;    // transmission functions (chunk, batch, n1, n2), or null
     int32_t* order;   // spectrum-pass molecule slots per slice, or null (identity)
     int64_t* mol_off;
     int64_t* elem_off;
@@ -1537,6 +1623,7 @@ struct FusedWorkspace {
     uint32_t* block_sums;
     float2* Y;
     float2* wave;
+    float2* carry;    // (batch): rounding rests of the waves' means (pass B)
     // water fill (emsim_hip_simulate_water): dense count planes and half
     // spectra of one slice of every molecule, per-molecule seeds
     float* hist;
@@ -1561,6 +1648,7 @@ struct WaterFill {
 FusedWorkspace fused_layout(const emsim_hip_slice_builder* b, int batch, int64_t n_atoms,
                             bool own_wave, char* base, bool water = false, bool raw = false) {
     FusedWorkspace w;
+    w.chunk = water ? 1 : fused_chunk(b, batch);
     w.n_rows = (int64_t)batch * b->n_slices * b->n_elems * b->n1;
     const int64_t n_scan = w.n_rows + 1;
     const int64_t n_blocks = ceil_div(n_scan, kScanTile);
@@ -1578,12 +1666,19 @@ FusedWorkspace fused_layout(const emsim_hip_slice_builder* b, int batch, int64_t
     w.row_start = (uint32_t*)(base + off); off += align_up(sizeof(uint32_t) * (size_t)n_scan);
     w.block_sums = (uint32_t*)(base + off); off += align_up(sizeof(uint32_t) * (size_t)n_blocks);
     w.Y = (float2*)(base + off);
-    off += align_up(sizeof(float2) * (size_t)batch * b->n1 * ldh);
+    off += align_up(sizeof(float2) * (size_t)w.chunk * batch * b->n1 * ldh);
+    w.phase = nullptr;
+    if (!water && fused_split(b, batch)) {
+        w.phase = (float2*)(base + off);
+        off += align_up(sizeof(float2) * (size_t)w.chunk * batch * b->n1 * b->n2);
+    }
     w.wave = nullptr;
     if (own_wave) {
         w.wave = (float2*)(base + off);
         off += align_up(sizeof(float2) * (size_t)batch * b->n1 * b->n2);
     }
+    w.carry = (float2*)(base + off);
+    off += align_up(sizeof(float2) * (size_t)batch);
     w.hist = nullptr;
     w.X = nullptr;
     w.seeds = nullptr;
@@ -1886,6 +1981,7 @@ int simulate_core(const emsim_hip_slice_builder* b, const emsim_hip_wave_propaga
     // others).  The last pass B runs every tile.
     ColDead dead = dead_columns(prop);
     dead.skip_tiles = true;
+    dead.carry = ws.carry;
     ColDead dead_last = dead;
     dead_last.skip_tiles = false;
     if (dead.lo <= dead.hi) {
@@ -1895,14 +1991,27 @@ int simulate_core(const emsim_hip_slice_builder* b, const emsim_hip_wave_propaga
     }
     for (int sl = 0; sl < b->n_slices; ++sl) {
         const bool last = sl == b->n_slices - 1;
+        dead.carry_first = dead_last.carry_first = sl == 0;
         if (!water.on) {
-            rc = spec_sparse(b->n1, ws.row_start, ws.bucket, b->sf, b->sf_tiles, ws.Y, sl,
-                             b->n_slices,
-                             b->n_elems, b->H, ldh, b->n2, symmetric_bandlimit ? 1 : 0, r * r,
-                             inv_npix, batch, order, b->tw, s);
-            if (rc) return rc;
-            rc = slice_pass_a(b->n2, sl == 0, ws.Y, wave, rows / 2, ldh, psi0, w->factor,
-                              slices_out, sl, b->n_slices, b->n1, dead, b->tw, s);
+            const int sc = sl % ws.chunk;   // plane of this slice in its chunk
+            if (sc == 0) {
+                const int n_sc = std::min(ws.chunk, b->n_slices - sl);
+                rc = spec_sparse(b->n1, ws.row_start, ws.bucket, b->sf, b->sf_tiles, ws.Y, sl,
+                                 n_sc, b->n_slices, b->n_elems, b->H, ldh, b->n2,
+                                 symmetric_bandlimit ? 1 : 0, r * r, inv_npix, batch, order,
+                                 b->tw, s);
+                if (!rc && ws.phase)
+                    rc = phase_rows(b->n2, ws.Y, ws.phase, n_sc, batch, b->n1, ldh, w->factor,
+                                    slices_out, sl, b->n_slices, b->tw, s);
+                if (rc) return rc;
+            }
+            if (ws.phase)
+                rc = phase_apply(b->n2, sl == 0, ws.phase + sc * batch * npix, wave, rows, psi0,
+                                 dead, b->tw, s);
+            else
+                rc = slice_pass_a(b->n2, sl == 0, ws.Y + (int64_t)sc * rows * ldh, wave, rows / 2,
+                                  ldh, psi0, w->factor, slices_out, sl, b->n_slices, b->n1, dead,
+                                  b->tw, s);
             if (rc) return rc;
         } else {
             // water: dense count planes of this slice (atoms + water), then

@@ -23,15 +23,21 @@ constexpr int kTwN = 4096;   // twiddle table length == largest supported N
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+// Every multiply-add of the transforms and of the pointwise steps between
+// them is written as fmaf, so no rounding is left to the compiler's choice of
+// contractions: the same value goes through the same roundings in whichever
+// kernel computes it (the batched path picks its kernels by the batch's size).
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+    return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
 }
+
+__device__ __forceinline__ float norm2(float2 a) { return fmaf(a.x, a.x, a.y * a.y); }
 
 // a * w (forward) or a * conj(w) (inverse)
 template <bool INV>
 __device__ __forceinline__ float2 mul_tw(float2 a, float2 w) {
-    if constexpr (!INV) return make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x);
-    else return make_float2(a.x * w.x + a.y * w.y, a.y * w.x - a.x * w.y);
+    if constexpr (!INV) return cmul(a, w);
+    else return make_float2(fmaf(a.x, w.x, a.y * w.y), fmaf(a.y, w.x, -(a.x * w.y)));
 }
 
 // a * (-i) forward, a * (+i) inverse
@@ -67,19 +73,24 @@ __device__ __forceinline__ void dft8(float2* a) {
     float2 o0 = a[1], o1 = a[3], o2 = a[5], o3 = a[7];
     dft4<INV>(e0, e1, e2, e3);
     dft4<INV>(o0, o1, o2, o3);
+    // o1, o3 times e^{-+i pi/4}, e^{-+3i pi/4}: the factor c goes into the last
+    // butterflies' multiply-adds
     const float c = 0.707106781186547524f;
+    float2 p1, p3;
     if constexpr (!INV) {
-        o1 = make_float2(c * (o1.x + o1.y), c * (o1.y - o1.x));     // * e^{-i pi/4}
-        o3 = make_float2(c * (o3.y - o3.x), -c * (o3.x + o3.y));    // * e^{-3i pi/4}
+        p1 = make_float2(o1.x + o1.y, o1.y - o1.x);
+        p3 = make_float2(o3.y - o3.x, -(o3.x + o3.y));
     } else {
-        o1 = make_float2(c * (o1.x - o1.y), c * (o1.x + o1.y));     // * e^{+i pi/4}
-        o3 = make_float2(-c * (o3.x + o3.y), c * (o3.x - o3.y));    // * e^{+3i pi/4}
+        p1 = make_float2(o1.x - o1.y, o1.x + o1.y);
+        p3 = make_float2(-(o3.x + o3.y), o3.x - o3.y);
     }
     o2 = mul_mi<INV>(o2);
     a[0] = cadd(e0, o0); a[4] = csub(e0, o0);
-    a[1] = cadd(e1, o1); a[5] = csub(e1, o1);
+    a[1] = make_float2(fmaf(c, p1.x, e1.x), fmaf(c, p1.y, e1.y));
+    a[5] = make_float2(fmaf(-c, p1.x, e1.x), fmaf(-c, p1.y, e1.y));
     a[2] = cadd(e2, o2); a[6] = csub(e2, o2);
-    a[3] = cadd(e3, o3); a[7] = csub(e3, o3);
+    a[3] = make_float2(fmaf(c, p3.x, e3.x), fmaf(c, p3.y, e3.y));
+    a[7] = make_float2(fmaf(-c, p3.x, e3.x), fmaf(-c, p3.y, e3.y));
 }
 
 template <int R, bool INV>
@@ -178,9 +189,13 @@ __device__ __forceinline__ float2 tw_get(const TwLds<N>& c, int q, int r, int k)
 // y[(j/Ns) Ns R + j%Ns + r Ns].
 // SYNC2: the barrier after the reads, which keeps the next pass's writes off
 // planes still being read; a caller that alternates two plane sets drops it.
+// dc (last pass, thread 0 only, null elsewhere): X[0]'s last sum, of R values,
+// in float64, with *dc added to it; *dc receives what its rounding to float32
+// leaves.
 template <int N, int EPT, int R, int Ns, bool INV, class TW, bool SYNC2 = true>
 __device__ __forceinline__ void stockham_pass(float2 (&v)[EPT], float* __restrict__ re,
-                                              float* __restrict__ im, int t, const TW& tw) {
+                                              float* __restrict__ im, int t, const TW& tw,
+                                              float2* dc = nullptr) {
     constexpr int NB = EPT / R;
     constexpr int S = N / EPT;
     constexpr bool LAST = (Ns * R == N);
@@ -196,7 +211,19 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[EPT], float* __restric
 #pragma unroll
             for (int r = 1; r < R; ++r) a[r] = mul_tw<INV>(a[r], tw_get<N, EPT, Ns, R>(tw, q, r, k));
         }
+        float2 sum = make_float2(0.f, 0.f);
+        if (LAST && q == 0 && dc) {
+            double sx = (double)dc->x, sy = (double)dc->y;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                sx += (double)a[r].x;
+                sy += (double)a[r].y;
+            }
+            sum = make_float2((float)sx, (float)sy);
+            *dc = make_float2((float)(sx - (double)sum.x), (float)(sy - (double)sum.y));
+        }
         dft<R, INV>(a);
+        if (LAST && q == 0 && dc) a[0] = sum;
         if constexpr (LAST) {
 #pragma unroll
             for (int r = 0; r < R; ++r) v[q + r * NB] = a[r];
@@ -225,10 +252,10 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[EPT], float* __restric
 
 template <int N, int EPT, int Ns, bool INV, class TW>
 __device__ __forceinline__ void fft_rest(float2 (&v)[EPT], float* re, float* im, int t,
-                                         const TW& tw) {
+                                         const TW& tw, float2* dc) {
     if constexpr (Ns < N) {
-        stockham_pass<N, EPT, 8, Ns, INV>(v, re, im, t, tw);
-        fft_rest<N, EPT, Ns * 8, INV>(v, re, im, t, tw);
+        stockham_pass<N, EPT, 8, Ns, INV>(v, re, im, t, tw, dc);
+        fft_rest<N, EPT, Ns * 8, INV>(v, re, im, t, tw, dc);
     }
 }
 
@@ -237,11 +264,11 @@ constexpr int fft_exchanges(int n) { return (ilog2(n) - ilog2(lead_radix(n))) / 
 
 template <int N, int EPT, int Ns, bool INV, int PASS, class TW>
 __device__ __forceinline__ void fft_rest_db(float2 (&v)[EPT], float* re0, float* im0, float* re1,
-                                            float* im1, int t, const TW& tw) {
+                                            float* im1, int t, const TW& tw, float2* dc) {
     if constexpr (Ns < N) {
         stockham_pass<N, EPT, 8, Ns, INV, TW, false>(v, PASS % 2 ? re1 : re0,
-                                                     PASS % 2 ? im1 : im0, t, tw);
-        fft_rest_db<N, EPT, Ns * 8, INV, PASS + 1>(v, re0, im0, re1, im1, t, tw);
+                                                     PASS % 2 ? im1 : im0, t, tw, dc);
+        fft_rest_db<N, EPT, Ns * 8, INV, PASS + 1>(v, re0, im0, re1, im1, t, tw, dc);
     }
 }
 
@@ -252,25 +279,25 @@ __device__ __forceinline__ void fft_rest_db(float2 (&v)[EPT], float* re0, float*
 // passes only once its reads of that set are done.
 template <int N, int EPT, bool INV, class TW>
 __device__ __forceinline__ void fft_n_db(float2 (&v)[EPT], float* re0, float* im0, float* re1,
-                                         float* im1, int t, const TW& tw) {
+                                         float* im1, int t, const TW& tw, float2* dc = nullptr) {
     static_assert(fft_exchanges(N) % 2 == 0, "alternating planes need an even exchange count");
     constexpr int R0 = lead_radix(N);
-    stockham_pass<N, EPT, R0, 1, INV, TW, false>(v, re0, im0, t, tw);
-    fft_rest_db<N, EPT, R0, INV, 1>(v, re0, im0, re1, im1, t, tw);
+    stockham_pass<N, EPT, R0, 1, INV, TW, false>(v, re0, im0, t, tw, dc);
+    fft_rest_db<N, EPT, R0, INV, 1>(v, re0, im0, re1, im1, t, tw, dc);
 }
 
 // Unnormalised length-N DFT of the values held by the N/EPT threads of one
 // row/column group.  Every thread of the block must call it (it contains
 // block barriers when N > 8).  tw is the twiddle table (const float2*) or
-// this thread's TwCache<N, EPT>.
+// this thread's TwCache<N, EPT>.  dc: see stockham_pass.
 template <int N, int EPT, bool INV, class TW>
 __device__ __forceinline__ void fft_n(float2 (&v)[EPT], float* re, float* im, int t,
-                                      const TW& tw) {
+                                      const TW& tw, float2* dc = nullptr) {
     static_assert(N >= 8 && N <= kTwN && (N & (N - 1)) == 0, "unsupported FFT length");
     static_assert(EPT >= 8 && EPT % 8 == 0 && EPT <= N, "EPT must be a multiple of 8");
     constexpr int R0 = lead_radix(N);
-    stockham_pass<N, EPT, R0, 1, INV>(v, re, im, t, tw);
-    fft_rest<N, EPT, R0, INV>(v, re, im, t, tw);
+    stockham_pass<N, EPT, R0, 1, INV>(v, re, im, t, tw, dc);
+    fft_rest<N, EPT, R0, INV>(v, re, im, t, tw, dc);
 }
 
 // ---------------------------------------------------------------------------

@@ -169,8 +169,8 @@ __global__ __launch_bounds__(256) void k_half_spectrum_sum(float2* __restrict__ 
         for (int e = 0; e < n_elems; ++e) {
             const float2 x = X[((int64_t)e * sc + s) * plane + (int64_t)i * ldh + j];
             const float f = sf[((int64_t)e * n1 + i) * H + j];
-            acc.x += x.x * f;
-            acc.y += x.y * f;
+            acc.x = fmaf(x.x, f, acc.x);
+            acc.y = fmaf(x.y, f, acc.y);
         }
         float m = inv_npix;
         if (bandlimit) {

@@ -5,7 +5,8 @@
 //   1. k_csr_classify / scan / k_csr_scatter: the atoms' exact bins (same
 //      edge tables and rule as the histogram kernels) are sorted into rows
 //      r = ((b nS + s) nE + e) n1 + x; row r's bucket holds the y bins.
-// Per slice s (three launches for the whole batch):
+// Per slice s (three launches for the whole batch; the first one, which does
+// not depend on the wave, takes several slices at once where they fit):
 //   2. k_spec_sparse (column tiles):  R_e(x, j) = sum_{atoms in row x} w^(j y)
 //      is the row DFT of the element's histogram plane, formed directly from
 //      the bucket; then FFT_col, * F_e, sum over e, * D / nPix, IFFT_col
@@ -234,8 +235,12 @@ __global__ void k_slice_order(const uint32_t* __restrict__ row_start, int n_slic
 
 // ---------------------------------------------------------------------------
 // Spectrum of one slice of every molecule, from the atom buckets.
-// One block per (column tile, molecule): a 1-D grid of n_tiles * batch.
-// Y rows are ldh complex apart, images n1 * ldh apart.
+// One block per (column tile, slice, molecule): a 1-D grid of n_tiles * n_sc *
+// batch for slices slice0 .. slice0 + n_sc - 1.  One slice of a small batch
+// fills a fraction of the chip for the whole latency of a block (18 us for 33
+// blocks of one 256^2 image), so a launch takes as many slices as its Y
+// planes' bound allows (fused_chunk).  Y is (n_sc, batch, n1, ldh): rows are
+// ldh complex apart.
 // ---------------------------------------------------------------------------
 // When the (molecule, slice)'s row table (n_elems * N + 1 entries), its atom
 // y-bins and the row twiddles (n2 entries) all fit, they are staged in LDS
@@ -485,8 +490,9 @@ template <int N>
 __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_SPEC_MIN_WAVES : 1) void k_spec_sparse(
     const uint32_t* __restrict__ row_start, const uint16_t* __restrict__ bucket,
     const float* __restrict__ sf, const float* __restrict__ sft, float2* __restrict__ Y,
-    int slice, int n_slices, int n_elems, int H, int ldh, int n2, int batch, int bandlimit,
-    int band_r2, float inv_npix, const int* __restrict__ order, const float2* __restrict__ tw) {
+    int slice0, int n_sc, int n_slices, int n_elems, int H, int ldh, int n2, int batch,
+    int bandlimit, int band_r2, float inv_npix, const int* __restrict__ order,
+    const float2* __restrict__ tw) {
     using Cfg = SpecCfg<N>;
     constexpr int EPT = Cfg::EPT;
     __shared__ float lds_re[Cfg::C * Cfg::STRIDE];
@@ -506,12 +512,19 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
     constexpr bool kTwCached = N <= 512 || N == 2048;
     __shared__ float2 lds_tw[kTwInLds ? N : 1];
     const unsigned item = spec_item(blockIdx.x, gridDim.x);
-    const int tile = (int)(item / (unsigned)batch);
+    // items: tile-major, then the launch's slices, then molecule slots
+    const unsigned per_tile = (unsigned)batch * (unsigned)n_sc;
+    const int tile = (int)(item / per_tile);
+    const unsigned plane_item = item % per_tile;
+    const int sc = (int)(plane_item / (unsigned)batch);
+    const int slice = slice0 + sc;
     // molecule slot -> molecule (null: identity).  Slots in order of the
     // slice's atom count, so each XCD's stream of blocks within a column
     // tile runs from the most expensive molecules to the cheapest.
-    const int bi = (int)(item % (unsigned)batch);
+    const int bi = (int)(plane_item % (unsigned)batch);
     const int b = order ? __builtin_amdgcn_readfirstlane(order[(int64_t)slice * batch + bi]) : bi;
+    // this (slice, molecule)'s half spectrum
+    Y += ((int64_t)sc * batch + b) * N * ldh;
     const int c = threadIdx.x % Cfg::C;
     const int t = threadIdx.x / Cfg::C;
     const int col = tile * Cfg::C + c;
@@ -528,7 +541,7 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
     const int sf_tiles = (H + Cfg::C - 1) / Cfg::C;   // tiles of the tile-major table
     // the packed lane parks each element's transform Z_e in padding column
     // H + e of its molecule's Y rows (ldh >= H + n_elems)
-    float2* zpark = Y + (int64_t)b * N * ldh + H;
+    float2* zpark = Y + H;
 
     // stage this (molecule, slice)'s rows (rows of all elements are adjacent),
     // its atoms' y bins and the twiddles.  The bucket range comes straight
@@ -689,8 +702,7 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
                     float2 wx;
                     if constexpr (kTwInLds) wx = lds_tw[p];
                     else wx = tw[p * (kTwN / N)];
-                    v[m].x += wx.x * wy.x - wx.y * wy.y;
-                    v[m].y += wx.x * wy.y + wx.y * wy.x;
+                    v[m] = cadd(v[m], cmul(wx, wy));
                 }
             }
         } else {
@@ -719,8 +731,8 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
         }
 #pragma unroll
         for (int m = 0; m < EPT; ++m) {
-            acc[m].x += v[m].x * fe[m];
-            acc[m].y += v[m].y * fe[m];
+            acc[m].x = fmaf(v[m].x, fe[m], acc[m].x);
+            acc[m].y = fmaf(v[m].y, fe[m], acc[m].y);
         }
         if (packed) {
 #pragma unroll
@@ -730,7 +742,7 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
     if (!any) {
         // empty slice of this molecule: the half spectrum is exactly zero
         if (valid) {
-            float2* dst = Y + (int64_t)b * N * ldh + col;
+            float2* dst = Y + col;
 #pragma unroll
             for (int m = 0; m < EPT; ++m) {
                 dst[(int64_t)(t + m * Cfg::T) * ldh] = make_float2(0.f, 0.f);
@@ -772,8 +784,8 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
                     const int64_t k1 = t + m * Cfg::T;
                     const float2 ze = zpark[k1 * ldh + e];
                     const float fq = fh[k1 * H];
-                    qa[m].x += ze.x * fq;
-                    qa[m].y += ze.y * fq;
+                    qa[m].x = fmaf(ze.x, fq, qa[m].x);
+                    qa[m].y = fmaf(ze.y, fq, qa[m].y);
                 }
             }
             const int kh = freq_int(half, n2);
@@ -810,7 +822,7 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
     }
     spec_fft<N, EPT, true, kTwCached>(acc, re, im, t, twc, tw);
     if (valid) {
-        float2* dst = Y + (int64_t)b * N * ldh + col;
+        float2* dst = Y + col;
         if (!packed) {
 #pragma unroll
             for (int m = 0; m < EPT; ++m) dst[(int64_t)(t + m * Cfg::T) * ldh] = acc[m];
@@ -830,6 +842,22 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
 // Pass A of one slice with the potential's C2R fused in: item = row pair
 // (image b, rows 2q, 2q+1).  FIRST: the incoming wave is the constant psi0.
 // ---------------------------------------------------------------------------
+// Hermitian extension of two half-spectrum rows (this thread's values at
+// k = t + m N/EPT), packed as a + i b for one complex inverse FFT whose real /
+// imaginary parts are the two rows' C2R.
+template <int N, int EPT>
+__device__ __forceinline__ void pack_c2r(const float2 (&ya)[EPT], const float2 (&yb)[EPT], int t,
+                                         float2 (&z)[EPT]) {
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+        const int k = t + m * (N / EPT);
+        float2 a = ya[m], b = yb[m];
+        if (k == 0 || k == N / 2) { a.y = 0.f; b.y = 0.f; }
+        if (k > N / 2) { a.y = -a.y; b.y = -b.y; }
+        z[m] = make_float2(a.x - b.y, a.y + b.x);
+    }
+}
+
 template <int N, bool FIRST>
 struct OpSlicePassA {
     static constexpr int T = RowCfg<N>::T, EPT = RowCfg<N>::EPT;
@@ -867,19 +895,6 @@ struct OpSlicePassA {
 #pragma unroll
         for (int m = 0; m < EPT; ++m) w[m] = ok ? src[t + m * T] : make_float2(0.f, 0.f);
     }
-    // Hermitian extension of both rows, packed as a + i b for one complex
-    // inverse FFT whose real / imaginary parts are the two rows' C2R.
-    __device__ __forceinline__ void pack(const float2 (&ya)[EPT], const float2 (&yb)[EPT], int t,
-                                         float2 (&z)[EPT]) const {
-#pragma unroll
-        for (int m = 0; m < EPT; ++m) {
-            const int k = t + m * T;
-            float2 a = ya[m], b = yb[m];
-            if (k == 0 || k == N / 2) { a.y = 0.f; b.y = 0.f; }
-            if (k > N / 2) { a.y = -a.y; b.y = -b.y; }
-            z[m] = make_float2(a.x - b.y, a.y + b.x);
-        }
-    }
     template <class TW>
     __device__ __forceinline__ void transmit_row(float2 (&w)[EPT], const float (&V)[EPT], int t,
                                                  float* re, float* im, const TW& tw) const {
@@ -893,8 +908,7 @@ struct OpSlicePassA {
         for (int m = 0; m < EPT; ++m) {
             float s, c;
             fast_sincos(__fmul_rn(V[m], factor), &s, &c);
-            const float2 x = w[m];
-            w[m] = make_float2(x.x * c - x.y * s, x.x * s + x.y * c);
+            w[m] = cmul(w[m], make_float2(c, s));
         }
         fft_n<N, EPT, false>(w, re, im, t, tw);
     }
@@ -969,7 +983,7 @@ __global__ __launch_bounds__(RowCfg<N>::BLOCK, EMSIM_PASSA_MIN_WAVES) void k_sli
         const bool ok = it < n_pairs;
         if constexpr (!FIRST) op.load_w(clamp(it), 1, t, true, w1);
         float2 z[EPT];
-        op.pack(ya, yb, t, z);
+        pack_c2r<N, EPT>(ya, yb, t, z);
         fft_n<N, EPT, true>(z, re, im, t, twc);
         float va[EPT], vb[EPT];
 #pragma unroll
@@ -986,6 +1000,123 @@ __global__ __launch_bounds__(RowCfg<N>::BLOCK, EMSIM_PASSA_MIN_WAVES) void k_sli
         op.transmit_row(w1, vb, t, re, im, twc);
         op.store_w(it, 1, t, ok, live, w1);
     }
+}
+
+// ---------------------------------------------------------------------------
+// Pass A in two kernels, for batches that leave most of the chip idle (the
+// rule is in fused_split): the potential's C2R and the transmission function
+// of a whole chunk of slices in one launch, then per slice only the wave's two
+// transforms, one row at a time.  The per-slice chain of dependent transforms
+// is then two long instead of five (C2R, and two per row of a pair).  Same
+// operations on the same values as k_slice_pass_a, so images don't depend on
+// which of the two a batch takes.
+// ---------------------------------------------------------------------------
+// Item = row pair of a (slice, molecule) plane: (cos, sin)(factor V) of both
+// rows, V clipped as in pass A (and written out if vout is given).
+template <int N>
+struct OpPhaseRows {
+    static constexpr int T = RowCfg<N>::T, EPT = RowCfg<N>::EPT;
+    const float2* Y;       // (n_sc, B, n1, ldh)
+    float2* phase;         // (n_sc, B, n1, N)
+    int ldh;
+    float factor;          // lambda * gamma
+    float* vout;           // nullable: potentials, (B, nS, n1, N)
+    int64_t v_img_stride;  // nS n1 N
+    int64_t v_slice_off;   // slice0 n1 N
+    int rows_per_img, batch;
+    struct Regs { float2 a[EPT], b[EPT]; };
+    __device__ __forceinline__ void load(int64_t pair, int t, bool, Regs& r) const {
+        const float2* ia = Y + pair * 2 * (int64_t)ldh;
+        const float2* ib = ia + ldh;
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            const int k = t + m * T;
+            const int kk = k <= N / 2 ? k : N - k;
+            r.a[m] = ia[kk];
+            r.b[m] = ib[kk];
+        }
+    }
+    template <class TW>
+    __device__ __forceinline__ void run(int64_t pair, int t, bool ok, Regs& r, float* re, float* im,
+                                        const TW& tw) const {
+        float2 z[EPT];
+        pack_c2r<N, EPT>(r.a, r.b, t, z);
+        fft_n<N, EPT, true>(z, re, im, t, tw);
+        if (!ok) return;
+        const int64_t row = pair * 2;
+        float2* pa = phase + row * N;
+        float* va = nullptr;
+        if (vout) {
+            const int64_t plane = row / rows_per_img, sc = plane / batch, img = plane - sc * batch;
+            va = vout + img * v_img_stride + v_slice_off +
+                 (sc * rows_per_img + (row - plane * rows_per_img)) * N;
+        }
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            const int k = t + m * T;
+            const float a = fmaxf(z[m].x, 1e-13f), b = fmaxf(z[m].y, 1e-13f);
+            float s, c;
+            fast_sincos(__fmul_rn(a, factor), &s, &c);
+            pa[k] = make_float2(c, s);
+            fast_sincos(__fmul_rn(b, factor), &s, &c);
+            pa[N + k] = make_float2(c, s);
+            if (va) {
+                va[k] = a;
+                va[N + k] = b;
+            }
+        }
+    }
+};
+
+// Item = wave row: IFFT_row (FIRST: the constant psi0) -> * phase -> FFT_row,
+// live columns stored (see OpSlicePassA).
+template <int N, bool FIRST>
+struct OpPhaseApply {
+    static constexpr int T = RowCfg<N>::T, EPT = RowCfg<N>::EPT;
+    const float2* phase;   // (B, n1, N) of this slice
+    float2* wave;
+    float psi0;
+    int dead_lo, dead_hi;
+    struct Regs { float2 w[EPT], p[EPT]; };
+    __device__ __forceinline__ void load(int64_t row, int t, bool, Regs& r) const {
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            if constexpr (!FIRST) r.w[m] = wave[row * N + t + m * T];
+            r.p[m] = phase[row * N + t + m * T];
+        }
+    }
+    template <class TW>
+    __device__ __forceinline__ void run(int64_t row, int t, bool ok, Regs& r, float* re, float* im,
+                                        const TW& tw) const {
+        if constexpr (FIRST) {
+#pragma unroll
+            for (int m = 0; m < EPT; ++m) r.w[m] = make_float2(psi0, 0.f);
+        } else {
+            fft_n<N, EPT, true>(r.w, re, im, t, tw);
+        }
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) r.w[m] = cmul(r.w[m], r.p[m]);
+        fft_n<N, EPT, false>(r.w, re, im, t, tw);
+        if (!ok) return;
+        float2* dst = wave + row * N;
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            const int k = t + m * T;
+            if (k < dead_lo || k > dead_hi) dst[k] = r.w[m];
+        }
+    }
+};
+
+template <int N>
+__global__ __launch_bounds__(RowCfg<N>::BLOCK) void k_phase_rows(OpPhaseRows<N> op, int64_t n,
+                                                                 int rpw, const float2* tw) {
+    row_worker<N>(op, n, rpw, tw);
+}
+template <int N, bool FIRST>
+__global__ __launch_bounds__(RowCfg<N>::BLOCK) void k_phase_apply(OpPhaseApply<N, FIRST> op,
+                                                                  int64_t n, int rpw,
+                                                                  const float2* tw) {
+    row_worker<N>(op, n, rpw, tw);
 }
 
 // Last slice of the fused path: propagator and lens in one multiplier.

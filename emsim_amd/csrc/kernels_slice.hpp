@@ -437,8 +437,8 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK) void k_col_spectrum(
 #pragma unroll
         for (int m = 0; m < Cfg::EPT; ++m) {
             const float fe = valid ? f[(int64_t)(t + m * Cfg::T) * H] : 0.f;
-            acc[m].x += v[m].x * fe;
-            acc[m].y += v[m].y * fe;
+            acc[m].x = fmaf(v[m].x, fe, acc[m].x);
+            acc[m].y = fmaf(v[m].y, fe, acc[m].y);
         }
     }
     // D(k1, j) / nPix: the reference's disk mask on integer frequencies

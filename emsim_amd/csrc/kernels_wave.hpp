@@ -96,7 +96,8 @@ struct LensMul {
         const float chi = __fsub_rn(__fmul_rn(__fmul_rn(c1, f2), f2), __fmul_rn(c2, f2));
         float s, c;
         fast_sincos(chi, &s, &c);
-        return make_float2((w.x * c + w.y * s) * inv_npix, (w.y * c - w.x * s) * inv_npix);
+        const float2 v = mul_tw<true>(w, make_float2(c, s));   // w exp(-i chi)
+        return make_float2(v.x * inv_npix, v.y * inv_npix);
     }
 };
 
@@ -258,8 +259,7 @@ struct OpTransmit {
         for (int m = 0; m < EPT; ++m) {
             float s, c;
             fast_sincos(__fmul_rn(r.p[m], factor), &s, &c);
-            const float2 w = r.v[m];
-            r.v[m] = make_float2(w.x * c - w.y * s, w.x * s + w.y * c);
+            r.v[m] = cmul(r.v[m], make_float2(c, s));
         }
         fft_n<N, EPT, false>(r.v, re, im, t, tw);
         if (ok) {
@@ -290,7 +290,7 @@ struct OpIfftIntensity {
         if (ok) {
             float* dst = img_out + it * N;
 #pragma unroll
-            for (int m = 0; m < EPT; ++m) dst[t + m * T] = r.v[m].x * r.v[m].x + r.v[m].y * r.v[m].y;
+            for (int m = 0; m < EPT; ++m) dst[t + m * T] = norm2(r.v[m]);
         }
     }
 };
@@ -386,8 +386,8 @@ constexpr int col_min_waves() {
 
 template <int N, class Mul, int SHAPE = 0>
 __global__ __launch_bounds__((ColCfg<N, SHAPE>::BLOCK), (col_min_waves<N, SHAPE>())) void k_col_fft_mul_ifft(
-    float2* data, int ld, int ncols, DeadCols dc, int64_t img_stride, int64_t n_tiles,
-    RunSched sched, Mul mul, const float2* __restrict__ tw) {
+    float2* data, int ld, int ncols, DeadCols dcols, int64_t img_stride, int64_t n_tiles,
+    RunSched sched, Mul mul, float2* carry, bool carry_first, const float2* __restrict__ tw) {
     using Cfg = ColCfg<N, SHAPE>;
     constexpr int EPT = Cfg::EPT;
     // a second plane set where the exchange count allows alternating sets
@@ -421,8 +421,8 @@ __global__ __launch_bounds__((ColCfg<N, SHAPE>::BLOCK), (col_min_waves<N, SHAPE>
         const uint32_t g0 = (uint32_t)(2 * (run_start + r) + parity);
         const bool tile_ok = g0 < (uint32_t)n_tiles;
         const uint32_t g = tile_ok ? g0 : (uint32_t)n_tiles - 1u;
-        const uint32_t img = g / (uint32_t)dc.live_per_img;
-        col = dc.tile((int)(g - img * (uint32_t)dc.live_per_img)) * Cfg::C + c;
+        const uint32_t img = g / (uint32_t)dcols.live_per_img;
+        col = dcols.tile((int)(g - img * (uint32_t)dcols.live_per_img)) * Cfg::C + c;
         ok = tile_ok && col < ncols;
         return data + (int64_t)img * img_stride + (col < ncols ? col : ncols - 1);
     };
@@ -443,12 +443,29 @@ __global__ __launch_bounds__((ColCfg<N, SHAPE>::BLOCK), (col_min_waves<N, SHAPE>
 #pragma unroll
         for (int m = 0; m < EPT; ++m) nxt[m] = base_n[(int64_t)(t + m * Cfg::T) * ld];
         // a dead column is zero after the propagator whatever it held
-        const bool dead = dc.dead(col);
+        const bool dead = dcols.dead(col);
 #pragma unroll
         for (int m = 0; m < EPT; ++m) cur[m] = dead ? make_float2(0.f, 0.f) : cur[m];
         const float2 py = mul.column(col);
-        if constexpr (DB) fft_n_db<N, EPT, false>(cur, re, im, re2, im2, t, twc);
-        else fft_n<N, EPT, false>(cur, re, im, t, twc);
+        // The wave's mean (bin 0 of column 0) is the image's scale, and its
+        // float32 rounding is one draw per slice that no average over pixels
+        // reduces.  Its last sum is done in float64, by one lane of the tiles
+        // that hold column 0, and what the rounding leaves is added to the
+        // next slice's sum (carry, one value per image), so the roundings
+        // don't add up along the slices.  Against 64 bits, 48 images of 256^2
+        // through 46 slices: rms error of the image's mean 6.9e-7 -> 2.0e-7,
+        // mean / largest image error 1.15e-6 / 2.0e-6 -> 1.01e-6 / 1.2e-6;
+        // 0.2 % of the time of 64 images of 512^2.
+        const bool dc = t == 0 && col == 0 && ok;
+        float2 rest = make_float2(0.f, 0.f);
+        float2* slot = nullptr;
+        if (dc && carry) {
+            slot = carry + (base - data) / img_stride;
+            if (!carry_first) rest = *slot;
+        }
+        if constexpr (DB) fft_n_db<N, EPT, false>(cur, re, im, re2, im2, t, twc, dc ? &rest : nullptr);
+        else fft_n<N, EPT, false>(cur, re, im, t, twc, dc ? &rest : nullptr);
+        if (slot) *slot = rest;
 #pragma unroll
         for (int m = 0; m < EPT; ++m) cur[m] = mul.apply(cur[m], t + m * Cfg::T, col, lds_px, py);
         if constexpr (DB) fft_n_db<N, EPT, true>(cur, re, im, re2, im2, t, twc);
@@ -489,16 +506,14 @@ __global__ void k_transmit(const float2* in, const float* __restrict__ V, float2
         const float pix = V[img * v_img_stride + (i - img * npix)];
         float s, c;
         fast_sincos(__fmul_rn(pix, factor), &s, &c);
-        const float2 w = in[i];
-        out[i] = make_float2(w.x * c - w.y * s, w.x * s + w.y * c);
+        out[i] = cmul(in[i], make_float2(c, s));
     }
 }
 
 __global__ void k_intensity(const float2* __restrict__ in, float* __restrict__ out, int64_t n) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const float2 w = in[i];
-        out[i] = w.x * w.x + w.y * w.y;
+        out[i] = norm2(in[i]);
     }
 }
 

@@ -1,0 +1,77 @@
+"""The batched path picks its kernels by the batch's size: slices per launch of
+the spectrum pass (up to a bound of plane memory) and pass A in one kernel or
+two (up to a bound of pixels).  Every choice runs the same operations on the
+same values, so a molecule's result is the same bits in any batch."""
+from ctypes import POINTER, c_int64
+
+import numpy as np
+import pytest
+import torch
+
+import emsim_amd
+from emsim_amd import synth
+from emsim_amd.backend import hip_ext
+from emsim_amd.backend._device import ptr, stream_handle
+from emsim_amd.backend.slice_builder_hip import MultiSlicesBuilder
+from emsim_amd.backend.wave_propagator_hip import WavePropagator
+from emsim_amd.batch import BatchPipe
+
+pytestmark = pytest.mark.gpu
+ELEMS = [1, 6, 7, 8, 16]
+SPLIT_PIXELS = 2 * 512 * 512   # the library's bound for pass A in two kernels
+
+
+def _tem():
+    return emsim_amd.tem.TEM(electron_dose=20, beam_energy_kev=200, cs_mm=1.3, defocus=700,
+                             aperture=10e-3)
+
+
+# (n, molecules beyond the bound, slices): one slice, fewer and more slices than
+# a launch takes (8 for the largest batch here, 19 at 128^2, all 40 alone)
+@pytest.mark.parametrize("n,over,slices", [(128, 1, 1), (128, 1, 40), (256, 1, 9),
+                                           (512, 1, 21), (64, 1, 3), (8, 1, 2)])
+def test_image_does_not_depend_on_the_batch(hip, n, over, slices):
+    batch = SPLIT_PIXELS // (n * n) + over
+    base = [synth.protein_cloud(400 + 150 * k, 40 + k) for k in range(4)]
+    pipe = BatchPipe(_tem(), 1.0, 2.0, n, slices, ELEMS)
+    prepared = [pipe.prepare(m) for m in base]
+    together = pipe.upload([prepared[k % 4] for k in range(batch)])
+    images = pipe.run(together)
+    waves, v = pipe.exit_waves_and_slices(together)
+    for k in range(4 if batch >= 4 else batch):
+        alone = pipe.upload([prepared[k]])
+        assert torch.equal(pipe.run(alone)[0], images[k])
+        w1, v1 = pipe.exit_waves_and_slices(alone)
+        assert torch.equal(w1[0], waves[k]) and torch.equal(v1[0], v[k])
+    assert torch.equal(images[batch - 1], images[(batch - 1) % 4])
+
+
+def test_rectangular_grid_does_not_depend_on_the_batch(hip):
+    """n1 != n2 (no band-limit disk), through the C ABI: rows and columns of
+    different length on both routes."""
+    n1, n2, slices = 128, 256, 5
+    builder = MultiSlicesBuilder(ELEMS, slices, n1, n2, 2.0, 1.0, 1.0).backend
+    prop = WavePropagator(n1, n2, 1.0, 1.0, 200.0).backend
+    square = BatchPipe(_tem(), 1.0, 2.0, 128, slices, ELEMS)
+    prepared = [square.prepare(synth.protein_cloud(500 + 100 * k, 60 + k)) for k in range(3)]
+
+    def run(batch):
+        out = torch.empty((len(batch), n1, n2), device="cuda")
+        n_atoms = batch.coords.shape[0]
+        need = hip_ext.raw("emsim_hip_simulate_workspace_size")(builder.h, len(batch), n_atoms, 0)
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        args = (builder.h, prop.h, ptr(batch.coords), n_atoms,
+                batch.mol_off.ctypes.data_as(POINTER(c_int64)),
+                batch.counts.ctypes.data_as(POINTER(c_int64)), len(batch), 4.5, 1.3, 700.0, 10e-3,
+                0, ptr(out), None, 0, ptr(ws))
+        # one byte less than the size function asks for is refused
+        rc = hip_ext.raw("emsim_hip_simulate")(*args, need - 1, stream_handle())
+        assert rc == hip_ext.EWORKSPACE
+        hip_ext.call("emsim_hip_simulate", *args, need, stream_handle())
+        return out
+
+    count = SPLIT_PIXELS // (n1 * n2) + 1
+    many = run(square.upload([prepared[k % 3] for k in range(count)]))
+    for k in range(3):
+        assert torch.equal(run(square.upload([prepared[k]]))[0], many[k])
+    assert np.isfinite(many.cpu().numpy()).all()
