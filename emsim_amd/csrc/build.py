@@ -25,7 +25,6 @@ FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-Wall",
     "-Wno-unused-function",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -42,17 +41,29 @@ def hipcc() -> str:
 def build(verbose: bool = False) -> Path:
     OUT_DIR.mkdir(parents=True, exist_ok=True)
     tmp = LIB.with_suffix(".so.tmp")
-    cmd = [hipcc(), *FLAGS, *map(str, SOURCES), "-o", str(tmp)]
     t0 = time.time()
+    objs = [OUT_DIR / (src.stem + ".o") for src in SOURCES]
+    cmds = [[hipcc(), *FLAGS, "-c", str(src), "-o", str(obj)] for src, obj in zip(SOURCES, objs)]
     if verbose:
-        print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
+        for cmd in cmds:
+            print(" ".join(cmd), flush=True)
+    procs = [subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+             for cmd in cmds]
+    outs = [proc.communicate()[0] for proc in procs]
+    for proc, out in zip(procs, outs):
+        if proc.returncode != 0:
+            sys.stderr.write(out)
+            raise RuntimeError(f"hipcc failed with exit code {proc.returncode}")
+    res = subprocess.run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs),
+                          "-o", str(tmp)], capture_output=True, text=True)
     if res.returncode != 0:
         sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError(f"hipcc failed with exit code {res.returncode}")
+        raise RuntimeError(f"hipcc link failed with exit code {res.returncode}")
+    for obj in objs:
+        obj.unlink()
     os.replace(tmp, LIB)
     if verbose:
-        noise = [ln for ln in res.stderr.splitlines() if "packed-fp32-ops" not in ln]
+        noise = [ln for out in outs for ln in out.splitlines() if "packed-fp32-ops" not in ln]
         if noise:
             print("\n".join(noise))
         print(f"built {LIB} in {time.time() - t0:.1f}s", flush=True)

@@ -113,10 +113,9 @@ bool size_supported(int n) { return pow2_supported(n) || chirp_supported(n); }
 // --------------------------------------------------------------------------
 struct ChirpPlan {
     int n = 0, M = 0;
-    float2* c_fwd = nullptr;   // (n) exp(-i pi m^2 / n)
-    float2* c_inv = nullptr;   // (n) conj
-    float2* b_fwd = nullptr;   // (M) FFT_M of conj(c_fwd) placed at m and M - m
-    float2* b_inv = nullptr;   // (M) the same for the inverse transform
+    float2* c = nullptr;   // (n) exp(-i pi m^2 / n)
+    float2* b = nullptr;   // (M) FFT_M of conj(c) placed at m and M - m, / M
+    ChirpTab tab() const { return ChirpTab{c, b, n}; }
 };
 
 // In-place iterative radix-2 FFT in float64, forward sign exp(-2 pi i j k / M).
@@ -143,7 +142,7 @@ void host_fft(std::vector<std::complex<double>>& a) {
 }
 
 void chirp_plan_free(ChirpPlan& p) {
-    for (float2** q : {&p.c_fwd, &p.c_inv, &p.b_fwd, &p.b_inv}) {
+    for (float2** q : {&p.c, &p.b}) {
         if (*q) (void)hipFree(*q);
         *q = nullptr;
     }
@@ -162,27 +161,22 @@ int chirp_plan_create(int n, ChirpPlan& p) {
         const long long q = ((long long)m * m) % (2LL * n);   // m^2 mod 2n: exact angle
         c[m] = std::polar(1.0, -pi * (double)q / (double)n);
     }
-    std::vector<float2> hc(n), hci(n), hb(M), hbi(M);
+    std::vector<float2> hc(n), hb(M);
+    for (int m = 0; m < n; ++m) hc[m] = make_float2((float)c[m].real(), (float)c[m].imag());
+    // the convolution kernel: conj of the transform's chirp, circular
+    std::vector<std::complex<double>> b(M, 0.0);
     for (int m = 0; m < n; ++m) {
-        hc[m] = make_float2((float)c[m].real(), (float)c[m].imag());
-        hci[m] = make_float2((float)c[m].real(), (float)-c[m].imag());
+        b[m] = std::conj(c[m]);
+        if (m > 0) b[M - m] = b[m];
     }
-    for (int dir = 0; dir < 2; ++dir) {
-        // the convolution kernel: conj of the transform's chirp, circular
-        std::vector<std::complex<double>> b(M, 0.0);
-        for (int m = 0; m < n; ++m) {
-            const std::complex<double> v = dir == 0 ? std::conj(c[m]) : c[m];
-            b[m] = v;
-            if (m > 0) b[M - m] = v;
-        }
-        host_fft(b);
-        std::vector<float2>& dst = dir == 0 ? hb : hbi;
-        for (int k = 0; k < M; ++k) dst[k] = make_float2((float)b[k].real(), (float)b[k].imag());
-    }
+    host_fft(b);
+    const double inv_m = 1.0 / (double)M;   // exact: M is a power of two
+    for (int k = 0; k < M; ++k)
+        hb[k] = make_float2((float)(b[k].real() * inv_m), (float)(b[k].imag() * inv_m));
     hipError_t err = hipSuccess;
-    const std::vector<float2>* src[4] = {&hc, &hci, &hb, &hbi};
-    float2** dst[4] = {&p.c_fwd, &p.c_inv, &p.b_fwd, &p.b_inv};
-    for (int i = 0; i < 4 && err == hipSuccess; ++i) {
+    const std::vector<float2>* src[2] = {&hc, &hb};
+    float2** dst[2] = {&p.c, &p.b};
+    for (int i = 0; i < 2 && err == hipSuccess; ++i) {
         err = hipMalloc(dst[i], src[i]->size() * sizeof(float2));
         if (err == hipSuccess)
             err = hipMemcpy(*dst[i], src[i]->data(), src[i]->size() * sizeof(float2),
@@ -306,11 +300,9 @@ struct emsim_hip_wave_propagator {
     float d1 = 0, d2 = 0, lam = 0, gamma = 0;
     float dfx = 0, dfy = 0, filter2 = 0, factor = 0;
     const float2* tw = nullptr;
-    // a wave shape that is not a power of two: chirp-z plans of both axes and
-    // the line buffer of one image (max(n1 M2, n2 M1) complex64)
+    // a wave shape that is not a power of two: chirp-z plans of both axes
     bool chirp = false;
     ChirpPlan p1, p2;
-    float2* work = nullptr;
 };
 
 // ==========================================================================
@@ -656,73 +648,194 @@ LensMul make_lens(const emsim_hip_wave_propagator* w, float cs_mm, float defocus
 }
 
 // --------------------------------------------------------------------------
-// chirp-z transforms of lines and images (sizes that are not powers of two)
+// chirp-z launches (sizes that are not powers of two), dispatched on the
+// convolution length M
 // --------------------------------------------------------------------------
-constexpr int64_t kOneImage = (int64_t)1 << 62;   // LineMap::per_img of a single image
+template <int M, int MODE>
+int launch_chirp_rows_mode(ChirpRows a, const float2* tw, hipStream_t s) {
+    static int resident_cache[64];
+    dim3 grid;
+    row_grid<M>(a.rows, a.rpb, grid,
+                resident_blocks(k_chirp_rows<M, MODE>, RowCfg<M>::BLOCK, resident_cache));
+    EMSIM_LAUNCH(M, (k_chirp_rows<M, MODE>), grid, dim3(RowCfg<M>::BLOCK), 0, s, a, tw);
+    return EMSIM_HIP_OK;
+}
+template <int M>
+int launch_chirp_rows(int mode, const ChirpRows& a, const float2* tw, hipStream_t s) {
+    if (mode == kChirpFwd) return launch_chirp_rows_mode<M, kChirpFwd>(a, tw, s);
+    if (mode == kChirpMid) return launch_chirp_rows_mode<M, kChirpMid>(a, tw, s);
+    if (mode == kChirpInv) return launch_chirp_rows_mode<M, kChirpInv>(a, tw, s);
+    return launch_chirp_rows_mode<M, kChirpInt>(a, tw, s);
+}
 
-// `lines` lines of p.n values (read from in through im in MODE, written to
-// out through om): their unnormalised DFT (inv: exp(+2 pi i j k / n)),
-// values k < n_out stored; real_out: real parts clipped at clip_lo.
-// work: lines x p.M complex64.
-int line_dft(const ChirpPlan& p, bool inv, int mode, const void* in, LineMap im, int64_t lines,
-             void* out, LineMap om, int n_out, bool real_out, float clip_lo, float2* work,
-             const float2* tw, hipStream_t s) {
-    if (lines <= 0) return EMSIM_HIP_OK;
-    const float2* c = inv ? p.c_inv : p.c_fwd;
-    const float2* B = inv ? p.b_inv : p.b_fwd;
-    const int64_t total = lines * (int64_t)p.M;
-    const dim3 gi(grid_for(total, 256)), blk(256);
-    if (mode == kReal)
-        EMSIM_LAUNCH(p.n, k_chirp_in<kReal>, gi, blk, 0, s, in, im, lines, p.n, p.M, c, work);
-    else if (mode == kHalf)
-        EMSIM_LAUNCH(p.n, k_chirp_in<kHalf>, gi, blk, 0, s, in, im, lines, p.n, p.M, c, work);
-    else
-        EMSIM_LAUNCH(p.n, k_chirp_in<kComplex>, gi, blk, 0, s, in, im, lines, p.n, p.M, c, work);
-    int rc = row_fft(p.M, false, work, work, lines, tw, s);
-    if (rc) return rc;
-    EMSIM_LAUNCH(p.n, k_line_mul, gi, blk, 0, s, work, lines, p.M, B);
-    rc = row_fft(p.M, true, work, work, lines, tw, s);
-    if (rc) return rc;
-    const float scale = 1.0f / (float)p.M;   // exact: M is a power of two
-    const dim3 go(grid_for(lines * (int64_t)n_out, 256));
-    if (real_out)
-        EMSIM_LAUNCH(p.n, k_chirp_out<true>, go, blk, 0, s, (const float2*)work, lines, n_out,
-                     p.M, c, scale, clip_lo, out, om);
-    else
-        EMSIM_LAUNCH(p.n, k_chirp_out<false>, go, blk, 0, s, (const float2*)work, lines, n_out,
-                     p.M, c, scale, clip_lo, out, om);
+// Narrow column tiles while the wide ones would not give every CU a block (one
+// 75^2 image of 20 slices: 222 us against 255; past it both measure the same).
+bool chirp_narrow(int64_t wide_tiles) { return wide_tiles < 256; }
+
+// Runs of n_tiles column tiles over at most one round of resident blocks.
+template <class K>
+int chirp_sched(K k, int block, int64_t n_tiles, int (&cache)[64], RunSched& sched, dim3& grid) {
+    if (n_tiles >= ((int64_t)1 << 31))
+        return fail(EMSIM_HIP_EINVAL, "chirp-z columns: %lld tiles, at most 2^31 - 1",
+                    (long long)n_tiles);
+    const int64_t resident = resident_blocks(k, block, cache);
+    const int64_t blocks = resident > 0 && resident < n_tiles ? resident : n_tiles;
+    sched = RunSched{(int)(n_tiles / blocks), (int)(n_tiles % blocks)};
+    grid = dim3((unsigned)blocks);
     return EMSIM_HIP_OK;
 }
 
-// Line maps of one n1 x n2 image with rows ld apart: its rows, its columns.
-LineMap rows_of(int ld) { return LineMap{kOneImage, 0, ld, 1}; }
-LineMap cols_of(int ld) { return LineMap{kOneImage, 0, 1, ld}; }
-
-// Unnormalised 2-D DFT of one n1 x n2 complex image (out may be in).
-int chirp_dft2(const emsim_hip_wave_propagator* w, bool inv, const float2* in, float2* out,
-               hipStream_t s) {
-    int rc = line_dft(w->p2, inv, kComplex, in, rows_of(w->n2), w->n1, out, rows_of(w->n2),
-                      w->n2, false, 0.f, w->work, w->tw, s);
+template <int M, class Mul, bool NARROW>
+int launch_chirp_cols_cfg(float2* data, int n_img, int n2, const ChirpTab& col, const Mul& mul,
+                          const float2* tw, hipStream_t s) {
+    using Cfg = ChirpColCfg<M, NARROW>;
+    static int resident_cache[64];
+    const int tiles = (int)ceil_div(n2, Cfg::C);
+    const int64_t n_tiles = (int64_t)tiles * n_img;
+    RunSched sched;
+    dim3 grid;
+    const int rc = chirp_sched(k_chirp_cols<M, Mul, NARROW>, Cfg::BLOCK, n_tiles, resident_cache,
+                               sched, grid);
     if (rc) return rc;
-    return line_dft(w->p1, inv, kComplex, out, cols_of(w->n2), w->n2, out, cols_of(w->n2),
-                    w->n1, false, 0.f, w->work, w->tw, s);
+    EMSIM_LAUNCH(M, (k_chirp_cols<M, Mul, NARROW>), grid, dim3(Cfg::BLOCK), 0, s, data, n2, tiles,
+                 n_tiles, sched, col, mul, tw);
+    return EMSIM_HIP_OK;
+}
+template <int M, class Mul>
+int launch_chirp_cols(float2* data, int n_img, int n2, const ChirpTab& col, const Mul& mul,
+                      const float2* tw, hipStream_t s) {
+    if (chirp_narrow(ceil_div(n2, ChirpColCfg<M, false>::C) * n_img))
+        return launch_chirp_cols_cfg<M, Mul, true>(data, n_img, n2, col, mul, tw, s);
+    return launch_chirp_cols_cfg<M, Mul, false>(data, n_img, n2, col, mul, tw, s);
 }
 
-// FFT -> Fourier-space multiplier -> IFFT of every image of a batch.
-template <class Mul>
-int chirp_filter(const emsim_hip_wave_propagator* w, const float2* in, float2* out, int batch,
-                 const Mul& mul, hipStream_t s) {
-    const int64_t npix = (int64_t)w->n1 * w->n2;
-    for (int b = 0; b < batch; ++b) {
-        float2* o = out + b * npix;
-        int rc = chirp_dft2(w, false, in + b * npix, o, s);
-        if (rc) return rc;
-        EMSIM_LAUNCH(0, k_spectrum_mul<Mul>, dim3(grid_for(npix, 256)), dim3(256), 0, s, o, npix,
-                     w->n1, w->n2, mul);
-        rc = chirp_dft2(w, true, o, o, s);
-        if (rc) return rc;
+template <int M>
+int launch_chirp_r2c(const float* hist, float2* X, int n_elems, int n_slices, int s0, int sc,
+                     int n1, int ldh, const ChirpTab& row, const float2* c1, const float2* tw,
+                     hipStream_t s) {
+    static int resident_cache[64];
+    const int64_t pairs = (int64_t)n_elems * sc * ((n1 + 1) / 2);
+    int rpb;
+    dim3 grid;
+    row_grid<M>(pairs, rpb, grid,
+                resident_blocks(k_chirp_r2c<M>, RowCfg<M>::BLOCK, resident_cache));
+    EMSIM_LAUNCH(M, (k_chirp_r2c<M>), grid, dim3(RowCfg<M>::BLOCK), 0, s, hist, X, n_elems,
+                 n_slices, s0, sc, n1, ldh, rpb, row, c1, tw);
+    return EMSIM_HIP_OK;
+}
+
+template <int M, bool NARROW>
+int launch_chirp_spectrum_cfg(float2* X, const float* sf, int n_elems, int sc, int H, int ldh,
+                              int n2, int bandlimit, int band_r2, float inv_npix,
+                              const ChirpTab& col, const float2* tw, hipStream_t s) {
+    using Cfg = ChirpColCfg<M, NARROW>;
+    static int resident_cache[64];
+    const int tiles = (int)ceil_div(H, Cfg::C);
+    RunSched sched;
+    dim3 grid;
+    const int rc = chirp_sched(k_chirp_spectrum<M, NARROW>, Cfg::BLOCK, (int64_t)tiles * sc,
+                               resident_cache, sched, grid);
+    if (rc) return rc;
+    EMSIM_LAUNCH(M, (k_chirp_spectrum<M, NARROW>), grid, dim3(Cfg::BLOCK), 0, s, X, sf, n_elems,
+                 sc, tiles, sched, H, ldh, n2, bandlimit, band_r2, inv_npix, col, tw);
+    return EMSIM_HIP_OK;
+}
+template <int M>
+int launch_chirp_spectrum(float2* X, const float* sf, int n_elems, int sc, int H, int ldh, int n2,
+                          int bandlimit, int band_r2, float inv_npix, const ChirpTab& col,
+                          const float2* tw, hipStream_t s) {
+    if (chirp_narrow(ceil_div(H, ChirpColCfg<M, false>::C) * sc))
+        return launch_chirp_spectrum_cfg<M, true>(X, sf, n_elems, sc, H, ldh, n2, bandlimit,
+                                                  band_r2, inv_npix, col, tw, s);
+    return launch_chirp_spectrum_cfg<M, false>(X, sf, n_elems, sc, H, ldh, n2, bandlimit, band_r2,
+                                               inv_npix, col, tw, s);
+}
+
+template <int M>
+int launch_chirp_c2r(const float2* X, float* out, int64_t rows, int ldh, float clip_lo,
+                     const ChirpTab& row, const float2* tw, hipStream_t s) {
+    static int resident_cache[64];
+    int rpb;
+    dim3 grid;
+    row_grid<M>((rows + 1) / 2, rpb, grid,
+                resident_blocks(k_chirp_c2r<M>, RowCfg<M>::BLOCK, resident_cache));
+    EMSIM_LAUNCH(M, (k_chirp_c2r<M>), grid, dim3(RowCfg<M>::BLOCK), 0, s, X, out, rows, ldh, rpb,
+                 clip_lo, row, tw);
+    return EMSIM_HIP_OK;
+}
+
+#define EMSIM_CHIRP_DISPATCH(M, FN, ...)                                             \
+    switch (M) {                                                                     \
+        case 16: return FN<16>(__VA_ARGS__);                                         \
+        case 32: return FN<32>(__VA_ARGS__);                                         \
+        case 64: return FN<64>(__VA_ARGS__);                                         \
+        case 128: return FN<128>(__VA_ARGS__);                                       \
+        case 256: return FN<256>(__VA_ARGS__);                                       \
+        case 512: return FN<512>(__VA_ARGS__);                                       \
+        case 1024: return FN<1024>(__VA_ARGS__);                                     \
+        case 2048: return FN<2048>(__VA_ARGS__);                                     \
+        case 4096: return FN<4096>(__VA_ARGS__);                                     \
+        default: return fail(EMSIM_HIP_EUNSUPPORTED, "unsupported chirp-z length %d", M); \
     }
-    return EMSIM_HIP_OK;
+
+int chirp_rows(int M, int mode, const ChirpRows& a, const float2* tw, hipStream_t s) {
+    EMSIM_CHIRP_DISPATCH(M, launch_chirp_rows, mode, a, tw, s);
+}
+int chirp_cols(int M, float2* data, int n_img, int n2, const ChirpTab& col, const PropagatorMul& mul,
+               const float2* tw, hipStream_t s) {
+    EMSIM_CHIRP_DISPATCH(M, launch_chirp_cols, data, n_img, n2, col, mul, tw, s);
+}
+int chirp_cols(int M, float2* data, int n_img, int n2, const ChirpTab& col, const LensMul& mul,
+               const float2* tw, hipStream_t s) {
+    EMSIM_CHIRP_DISPATCH(M, launch_chirp_cols, data, n_img, n2, col, mul, tw, s);
+}
+int chirp_r2c(int M, const float* hist, float2* X, int n_elems, int n_slices, int s0, int sc, int n1,
+              int ldh, const ChirpTab& row, const float2* c1, const float2* tw, hipStream_t s) {
+    EMSIM_CHIRP_DISPATCH(M, launch_chirp_r2c, hist, X, n_elems, n_slices, s0, sc, n1, ldh, row, c1,
+                         tw, s);
+}
+int chirp_spectrum(int M, float2* X, const float* sf, int n_elems, int sc, int H, int ldh, int n2,
+                   int bandlimit, int band_r2, float inv_npix, const ChirpTab& col,
+                   const float2* tw, hipStream_t s) {
+    EMSIM_CHIRP_DISPATCH(M, launch_chirp_spectrum, X, sf, n_elems, sc, H, ldh, n2, bandlimit,
+                         band_r2, inv_npix, col, tw, s);
+}
+int chirp_c2r(int M, const float2* X, float* out, int64_t rows, int ldh, float clip_lo,
+              const ChirpTab& row, const float2* tw, hipStream_t s) {
+    EMSIM_CHIRP_DISPATCH(M, launch_chirp_c2r, X, out, rows, ldh, clip_lo, row, tw, s);
+}
+
+// Row-pass arguments of a batch of waves (V: one slice's potentials, or null).
+ChirpRows chirp_row_args(const emsim_hip_wave_propagator* w, const float2* in, float2* out,
+                         int batch, const float* V, int64_t v_img_stride) {
+    ChirpRows a;
+    a.in = in;
+    a.out = out;
+    a.image = nullptr;
+    a.V = V;
+    a.v_img_stride = v_img_stride;
+    a.factor = w->factor;
+    a.rows = (int64_t)batch * w->n1;
+    a.rows_per_img = w->n1;
+    a.row = w->p2.tab();
+    a.c1 = w->p1.c;
+    a.rpb = 1;
+    return a;
+}
+
+// FFT -> Fourier-space multiplier -> IFFT of every image of a batch (out: the
+// wave, or with image set its intensity, out being scratch).
+template <class Mul>
+int chirp_filter(const emsim_hip_wave_propagator* w, const float2* in, float2* out, float* image,
+                 int batch, const Mul& mul, hipStream_t s) {
+    ChirpRows a = chirp_row_args(w, in, out, batch, nullptr, 0);
+    int rc = chirp_rows(w->p2.M, kChirpFwd, a, w->tw, s);
+    if (rc) return rc;
+    rc = chirp_cols(w->p1.M, out, batch, w->n2, w->p1.tab(), mul, w->tw, s);
+    if (rc) return rc;
+    a.in = out;
+    a.image = image;
+    return chirp_rows(w->p2.M, image ? kChirpInt : kChirpInv, a, w->tw, s);
 }
 
 }  // namespace
@@ -988,13 +1101,9 @@ extern "C" int emsim_hip_add_water(const emsim_hip_slice_builder* b, float* hist
 
 namespace {
 // Workspace of make_slices per slice of a chunk: the half spectra of every
-// element, plus (chirp-z sizes) the line buffer of one element's transforms.
+// element.
 size_t slices_bytes_per_slice(const emsim_hip_slice_builder* b) {
-    size_t per = (size_t)b->n_elems * b->n1 * half_ld(b->H) * sizeof(float2);
-    if (b->chirp)
-        per += sizeof(float2) * (size_t)std::max((int64_t)b->n1 * b->p2.M,
-                                                 (int64_t)b->H * b->p1.M);
-    return per;
+    return (size_t)b->n_elems * b->n1 * half_ld(b->H) * sizeof(float2);
 }
 }  // namespace
 
@@ -1026,35 +1135,18 @@ extern "C" int emsim_hip_make_slices(const emsim_hip_slice_builder* b, const flo
     const int r = (b->n1 < b->n2 ? b->n1 : b->n2) / 2;
     const float inv_npix = 1.0f / (float)((int64_t)b->n1 * b->n2);
     if (b->chirp) {
-        // the same passes through chirp-z transforms: R2C rows, column DFTs,
-        // spectrum sum, inverse column DFTs, C2R rows with the clip
-        float2* work = X + (size_t)b->n_elems * chunk * b->n1 * ldh;
-        const int n1 = b->n1, n2 = b->n2, H = b->H, nE = b->n_elems;
+        // the same passes through chirp-z transforms
         for (int s0 = 0; s0 < b->n_slices; s0 += chunk) {
             const int sc = (b->n_slices - s0) < chunk ? (b->n_slices - s0) : chunk;
-            for (int e = 0; e < nE; ++e) {
-                float2* Xe = X + (size_t)e * sc * n1 * ldh;
-                const float* in = hist + ((int64_t)e * b->n_slices + s0) * n1 * n2;
-                int rc = line_dft(b->p2, false, kReal, in, rows_of(n2), (int64_t)sc * n1, Xe,
-                                  rows_of(ldh), H, false, 0.f, work, b->tw, s);
-                if (rc) return rc;
-                // columns of sc images (n1 rows of ldh) of this element
-                const LineMap cm{H, (int64_t)n1 * ldh, 1, ldh};
-                rc = line_dft(b->p1, false, kComplex, Xe, cm, (int64_t)sc * H, Xe, cm, n1,
-                              false, 0.f, work, b->tw, s);
-                if (rc) return rc;
-            }
-            const int64_t total = (int64_t)sc * n1 * H;
-            EMSIM_LAUNCH(0, k_half_spectrum_sum, dim3(grid_for(total, 256)), dim3(256), 0, s, X,
-                         b->sf, nE, sc, n1, H, ldh, n2, symmetric_bandlimit ? 1 : 0, r * r,
-                         inv_npix);
-            const LineMap cm{H, (int64_t)n1 * ldh, 1, ldh};
-            int rc = line_dft(b->p1, true, kComplex, X, cm, (int64_t)sc * H, X, cm, n1, false,
-                              0.f, work, b->tw, s);
+            int rc = chirp_r2c(b->p2.M, hist, X, b->n_elems, b->n_slices, s0, sc, b->n1, ldh,
+                               b->p2.tab(), b->p1.c, b->tw, s);
             if (rc) return rc;
-            rc = line_dft(b->p2, true, kHalf, X, rows_of(ldh), (int64_t)sc * n1,
-                          out + (int64_t)s0 * n1 * n2, rows_of(n2), n2, true, 1e-13f, work,
-                          b->tw, s);
+            rc = chirp_spectrum(b->p1.M, X, b->sf, b->n_elems, sc, b->H, ldh, b->n2,
+                                symmetric_bandlimit ? 1 : 0, r * r, inv_npix, b->p1.tab(), b->tw,
+                                s);
+            if (rc) return rc;
+            rc = chirp_c2r(b->p2.M, X, out + (int64_t)s0 * b->n1 * b->n2, (int64_t)sc * b->n1, ldh,
+                           1e-13f, b->p2.tab(), b->tw, s);
             if (rc) return rc;
         }
         return EMSIM_HIP_OK;
@@ -1110,12 +1202,6 @@ extern "C" int emsim_hip_wave_propagator_create(emsim_hip_wave_propagator** out,
         w->chirp = true;
         rc = chirp_plan_create(n1, w->p1);
         if (!rc) rc = chirp_plan_create(n2, w->p2);
-        if (!rc) {
-            const int64_t lines = std::max((int64_t)n1 * w->p2.M, (int64_t)n2 * w->p1.M);
-            if (hipMalloc(&w->work, sizeof(float2) * (size_t)lines) != hipSuccess)
-                rc = fail(EMSIM_HIP_ENOMEM, "wave_propagator_create: no device memory for "
-                                            "the chirp-z line buffer");
-        }
     }
     if (rc) {
         emsim_hip_wave_propagator_destroy(w);
@@ -1129,7 +1215,6 @@ extern "C" int emsim_hip_wave_propagator_destroy(emsim_hip_wave_propagator* w) {
     if (!w) return EMSIM_HIP_OK;
     chirp_plan_free(w->p1);
     chirp_plan_free(w->p2);
-    if (w->work) (void)hipFree(w->work);
     delete w;
     return EMSIM_HIP_OK;
 }
@@ -1163,7 +1248,8 @@ extern "C" int emsim_hip_space_propagate(const emsim_hip_wave_propagator* w, con
     if (!w || !wave || !out || batch < 1) return fail(EMSIM_HIP_EINVAL, "space_propagate: bad arguments");
     if (batch > 65535) return fail(EMSIM_HIP_EUNSUPPORTED, "space_propagate: batch <= 65535");
     if (w->chirp)
-        return chirp_filter(w, (const float2*)wave, (float2*)out, batch, make_propagator(w, dz), s);
+        return chirp_filter(w, (const float2*)wave, (float2*)out, nullptr, batch,
+                            make_propagator(w, dz), s);
     const int64_t rows = (int64_t)batch * w->n1;
     const int64_t npix = (int64_t)w->n1 * w->n2;
     float2* o = (float2*)out;
@@ -1187,20 +1273,17 @@ extern "C" int emsim_hip_multislice_propagate(const emsim_hip_wave_propagator* w
     const PropagatorMul prop = make_propagator(w, dz);
     float2* o = (float2*)out;
     if (w->chirp) {
-        // image by image: transmission, then the propagator through chirp-z
-        // transforms (WavePropagator.cpp:90-103)
-        for (int b = 0; b < batch; ++b) {
-            float2* ob = o + b * npix;
-            for (int sl = 0; sl < n_slices; ++sl) {
-                const float2* src = sl == 0 ? (const float2*)wave + b * npix : ob;
-                EMSIM_LAUNCH(0, k_transmit, dim3(grid_for(npix, 256)), dim3(256), 0, s, src,
-                             slices + b * slices_batch_stride + (int64_t)sl * npix, ob, npix, npix,
-                             (int64_t)0, w->factor);
-                const int rc = chirp_filter(w, ob, ob, 1, prop, s);
-                if (rc) return rc;
-            }
+        // WavePropagator.cpp:90-103; the wave stays chirped between the passes
+        ChirpRows a = chirp_row_args(w, (const float2*)wave, o, batch, slices, slices_batch_stride);
+        for (int sl = 0; sl < n_slices; ++sl) {
+            a.V = slices + (int64_t)sl * npix;
+            int rc = chirp_rows(w->p2.M, sl == 0 ? kChirpFwd : kChirpMid, a, w->tw, s);
+            if (rc) return rc;
+            a.in = o;
+            rc = chirp_cols(w->p1.M, o, batch, w->n2, w->p1.tab(), prop, w->tw, s);
+            if (rc) return rc;
         }
-        return EMSIM_HIP_OK;
+        return chirp_rows(w->p2.M, kChirpInv, a, w->tw, s);
     }
     for (int sl = 0; sl < n_slices; ++sl) {
         const float2* src = sl == 0 ? (const float2*)wave : o;
@@ -1220,7 +1303,7 @@ extern "C" int emsim_hip_lens_propagate(const emsim_hip_wave_propagator* w, cons
     if (!w || !wave || !out || batch < 1) return fail(EMSIM_HIP_EINVAL, "lens_propagate: bad arguments");
     if (batch > 65535) return fail(EMSIM_HIP_EUNSUPPORTED, "lens_propagate: batch <= 65535");
     if (w->chirp)
-        return chirp_filter(w, (const float2*)wave, (float2*)out, batch,
+        return chirp_filter(w, (const float2*)wave, (float2*)out, nullptr, batch,
                             make_lens(w, cs_mm, defocus, aperture), s);
     const int64_t rows = (int64_t)batch * w->n1;
     const int64_t npix = (int64_t)w->n1 * w->n2;
@@ -1244,14 +1327,9 @@ extern "C" int emsim_hip_lens_intensity(const emsim_hip_wave_propagator* w, cons
     const int64_t rows = (int64_t)batch * w->n1;
     const int64_t npix = (int64_t)w->n1 * w->n2;
     float2* o = (float2*)scratch;
-    if (w->chirp) {
-        const int rc = chirp_filter(w, (const float2*)wave, o, batch,
-                                    make_lens(w, cs_mm, defocus, aperture), s);
-        if (rc) return rc;
-        EMSIM_LAUNCH(0, k_intensity, dim3(grid_for(npix * batch, 256)), dim3(256), 0, s,
-                     (const float2*)o, image, npix * batch);
-        return EMSIM_HIP_OK;
-    }
+    if (w->chirp)
+        return chirp_filter(w, (const float2*)wave, o, image, batch,
+                            make_lens(w, cs_mm, defocus, aperture), s);
     int rc = row_fft(w->n2, false, (const float2*)wave, o, rows, w->tw, s);
     if (!rc)
         rc = col_lens(w->n1, o, w->n2, w->n2, npix, batch, make_lens(w, cs_mm, defocus, aperture),
