@@ -87,6 +87,9 @@ _SIGNATURES = {
                                        POINTER(c_int64), c_int, c_float, c_float, c_float,
                                        c_float, c_int, c_void_p, c_void_p, c_int, c_void_p,
                                        c_size_t, c_void_p]),
+    "emsim_hip_pack_raw": (c_int, [c_int, POINTER(c_void_p), POINTER(c_void_p),
+                                   POINTER(c_int64), c_void_p, c_int64, c_void_p, c_void_p,
+                                   c_void_p, c_int, POINTER(c_int)]),
     "emsim_hip_gemm": (c_int, [c_void_p, c_void_p]),
     "emsim_hip_fno_create": (c_int, [POINTER(c_void_p), c_int, c_int, c_int, c_int, c_int]),
     "emsim_hip_fno_destroy": (None, [c_void_p]),

