@@ -83,6 +83,11 @@ struct emsim_hip_fno {
     uint16_t* fx2 = nullptr;      // (2 M1, n)
     uint16_t* gx = nullptr;       // (2 n, 2 M1)
     uint16_t* gy = nullptr;       // (n, 2 M2)
+    // transposes, for the fused backward pass
+    uint16_t* fyt = nullptr;      // (n, 2 M2)
+    uint16_t* fx2t = nullptr;     // (n, 2 M1)
+    uint16_t* gxt = nullptr;      // (2 M1, 2 n)
+    uint16_t* gyt = nullptr;      // (2 M2, n)
 };
 
 namespace {
@@ -267,7 +272,17 @@ int emsim_hip_fno_create(emsim_hip_fno** out, int n, int in_channels, int channe
         if (hipMalloc(dst, src.size() * 2) != hipSuccess) return false;
         return hipMemcpy(*dst, src.data(), src.size() * 2, hipMemcpyHostToDevice) == hipSuccess;
     };
-    if (!upload(&f->fy, fy) || !upload(&f->fx2, fx2) || !upload(&f->gx, gx) || !upload(&f->gy, gy))
+    auto transposed = [](const std::vector<uint16_t>& a, size_t rows, size_t cols) {
+        std::vector<uint16_t> t(a.size());
+        for (size_t i = 0; i < rows; ++i)
+            for (size_t j = 0; j < cols; ++j) t[j * rows + i] = a[i * cols + j];
+        return t;
+    };
+    if (!upload(&f->fy, fy) || !upload(&f->fx2, fx2) || !upload(&f->gx, gx) || !upload(&f->gy, gy) ||
+        !upload(&f->fyt, transposed(fy, (size_t)2 * M2, n)) ||
+        !upload(&f->fx2t, transposed(fx2, (size_t)2 * M1, n)) ||
+        !upload(&f->gxt, transposed(gx, (size_t)2 * n, (size_t)2 * M1)) ||
+        !upload(&f->gyt, transposed(gy, n, (size_t)2 * M2)))
         return fail_free(EMSIM_HIP_EDEVICE, "basis upload failed");
     *out = f;
     return EMSIM_HIP_OK;
@@ -276,7 +291,8 @@ int emsim_hip_fno_create(emsim_hip_fno** out, int n, int in_channels, int channe
 void emsim_hip_fno_destroy(emsim_hip_fno* f) {
     if (!f) return;
     for (void* p : {(void*)f->params, (void*)f->grads, (void*)f->adam_m, (void*)f->adam_v,
-                    (void*)f->params16, (void*)f->fy, (void*)f->fx2, (void*)f->gx, (void*)f->gy})
+                    (void*)f->params16, (void*)f->fy, (void*)f->fx2, (void*)f->gx, (void*)f->gy,
+                    (void*)f->fyt, (void*)f->fx2t, (void*)f->gxt, (void*)f->gyt})
         if (p) (void)hipFree(p);
     delete f;
 }
@@ -564,6 +580,97 @@ int forward_fused(const emsim_hip_fno* f, const FnoWs& w, const void* x, float* 
     return EMSIM_HIP_OK;
 }
 
+// The fused backward pass: the fused rows' networks whose x-transforms fit
+// k_fno_xred / k_fno_xexp.
+bool fused_bwd_ok(const emsim_hip_fno* f, int batch) {
+    const int64_t nc = 2 * (int64_t)f->M2 * f->C;
+    return fused_rows_ok(f) && 2 * f->M1 <= 64 && 2 * f->M1 % 16 == 0 && nc % 128 == 0 &&
+           f->n % 32 == 0 &&
+           (int64_t)batch * (f->n / 32) * (nc / 128) <= 0x7fffffff;
+}
+
+template <int K2F, int SRC, bool LIFT, int K1F>
+int launch_bwd(const FnoBwdArgs& a, int blocks, hipStream_t s) {
+    EMSIM_LAUNCH(0, (k_fno_bwd_rows<K2F, SRC, LIFT, K1F>), dim3((unsigned)blocks),
+                 dim3(64 * kFnoBwdWaves), kFnoBwdLds(a.n, 16 * K2F), s, a);
+    return EMSIM_HIP_OK;
+}
+template <int K2F>
+int launch_bwd_rows(const FnoBwdArgs& a, int src, bool lift, int k1, int blocks, hipStream_t s) {
+    if (src == kBwdHead) return launch_bwd<K2F, kBwdHead, false, 2>(a, blocks, s);
+    if (!lift) return src == kBwdOut ? launch_bwd<K2F, kBwdOut, false, 2>(a, blocks, s)
+                                     : launch_bwd<K2F, kBwdDz, false, 2>(a, blocks, s);
+    if (k1 == 16) return src == kBwdOut ? launch_bwd<K2F, kBwdOut, true, 1>(a, blocks, s)
+                                        : launch_bwd<K2F, kBwdDz, true, 1>(a, blocks, s);
+    return src == kBwdOut ? launch_bwd<K2F, kBwdOut, true, 2>(a, blocks, s)
+                          : launch_bwd<K2F, kBwdDz, true, 2>(a, blocks, s);
+}
+
+int part_sum(const float* part, int np, const FnoGradDst& d, hipStream_t s) {
+    const int count = d.qw ? kFnoBwdPart : 1056;
+    EMSIM_LAUNCH(0, k_part_sum, dim3((unsigned)((count + 7) / 8)), dim3(256), 0, s, part, np, d);
+    return EMSIM_HIP_OK;
+}
+
+int backward_fused(emsim_hip_fno* f, const FnoWs& w, const void* x, const float* dout, int batch,
+                   hipStream_t s) {
+    const int n = f->n, C = f->C, M1 = f->M1, M2 = f->M2, L = f->L;
+    const int nc = 2 * M2 * C;
+    float* g = f->grads;
+    FnoBwdArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.dout = dout;
+    a.q16 = f->params16 + f->off_qw;
+    a.dz = w.dz;
+    a.vL = w.v[L];
+    a.fyt = f->fyt;
+    a.gyt = f->gyt;
+    a.dU = w.u;
+    a.part = w.dout_partial;
+    a.rows = (int64_t)batch * n;
+    a.n = n;
+    // one block of eight waves per CU (the bases fill its LDS), rows dealt out
+    // evenly
+    const int64_t waves = 256 * kFnoBwdWaves;
+    a.rpw = (int)((a.rows + waves - 1) / waves);
+    const int64_t per = (int64_t)a.rpw * kFnoBwdWaves;
+    const int blocks = (int)((a.rows + per - 1) / per);
+    int rc;
+    auto rows = [&](int src, bool lift) {
+        return M2 == 8 ? launch_bwd_rows<1>(a, src, lift, f->cin_pad, blocks, s)
+                       : launch_bwd_rows<2>(a, src, lift, f->cin_pad, blocks, s);
+    };
+    a.v = w.v[L - 1];
+    if ((rc = rows(kBwdHead, false))) return rc;
+    if ((rc = part_sum(w.dout_partial, blocks,
+                       FnoGradDst{g + f->off_w[L - 1], g + f->off_b[L - 1], g + f->off_qw,
+                                  g + f->off_qb, C * C},
+                       s)))
+        return rc;
+    for (int l = L - 1; l >= 0; --l) {
+        // the spectral branch: dU -> dOb -> (dR, dPQ) -> dT
+        EMSIM_LAUNCH(0, k_fno_xred, dim3((unsigned)(batch * (nc / 2 / 32))), dim3(256), 0, s, f->gxt,
+                     (const float*)w.u, w.ob, 2 * M1, 2 * n, nc / 2);
+        EMSIM_LAUNCH(0, k_fno_mix_bwd<32>, dim3(M1 * M2), dim3(256), 0, s, (const float*)w.pq[l],
+                     (const float2*)(f->params + f->off_r[l]), (const float*)w.ob,
+                     (float2*)(g + f->off_r[l]), w.pq[l], batch, M1, M2);
+        EMSIM_LAUNCH(0, k_fno_xexp, dim3((unsigned)(batch * (n / 32) * (nc / 128))), dim3(256), 0, s,
+                     f->fx2t, (const float*)w.pq[l], w.ty, n, 2 * M1, nc);
+        const bool lift = l == 0;
+        a.w16 = f->params16 + f->off_w[l];
+        a.dT = w.ty;
+        a.z = lift ? nullptr : w.z[l - 1];
+        a.v = lift ? (const uint16_t*)x : w.v[l - 1];
+        if ((rc = rows(l == L - 1 ? kBwdOut : kBwdDz, lift))) return rc;
+        const FnoGradDst d = lift ? FnoGradDst{g + f->off_lw, g + f->off_lb, nullptr, nullptr,
+                                               f->cin_pad * C}
+                                  : FnoGradDst{g + f->off_w[l - 1], g + f->off_b[l - 1], nullptr,
+                                               nullptr, C * C};
+        if ((rc = part_sum(w.dout_partial, blocks, d, s))) return rc;
+    }
+    return EMSIM_HIP_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -645,6 +752,8 @@ int emsim_hip_fno_backward(emsim_hip_fno* f, const void* x_dev, const float* dou
     if (workspace_bytes < w.bytes)
         return fail(EMSIM_HIP_EWORKSPACE, "fno_backward: workspace %zu < %zu", workspace_bytes, w.bytes);
     hipStream_t s = (hipStream_t)stream;
+    if (fused_bwd_ok(f, batch) && !g_fno_force_generic)
+        return backward_fused(f, w, x_dev, dout_dev, batch, s);
     const int n = f->n, C = f->C, M1 = f->M1, M2 = f->M2, L = f->L;
     const int64_t P = (int64_t)batch * n * n;
     float* g = f->grads;

@@ -900,6 +900,437 @@ __global__ __launch_bounds__(256) void k_fno_mix_bwd(const float* __restrict__ P
     }
 }
 
+// ---------------------------------------------------------------------------
+// Backward of the 32-channel network, fused per image row.  One wave per row,
+// walking its 32-pixel tiles in order; channels are the MFMA rows and pixels
+// its columns, as in k_fno_rows.  From dz_l, the gradient at layer l's
+// pre-activation, a launch computes
+//   dv = W_l dz_l + dT_l^T Fy          (the gradient at layer l's input)
+//   dz_(l-1) = dv gelu'(z_(l-1))       (stored over dz_l)
+//   db_(l-1) += dz, dW_(l-1) += v dz^T, dU_(l-1) = dz^T Gy per row
+// so each of dz, z and v crosses memory once per layer, where separate
+// activation, weight-gradient, column-sum and transform launches read dz five
+// times.  SRC: where dz comes from -- kBwdHead: dz of the last layer from the
+// loss gradient (dout Qw^T, no layer below), with dQw and dqb; kBwdOut: the
+// same dz as the source of a step; kBwdDz: the stored dz.  LIFT: the step below
+// is the lifting (no activation, v is the network's input, no transform).
+// float32 is rounded to bf16 exactly where k_gemm rounded its operands, and
+// the sums over a row's pixels run in the same order.
+// Bound by HBM: 384 bytes a pixel and middle layer, 193 us for 8 x 512^2 pixels
+// (4.2 TB/s); the whole backward pass of that batch 8.6 ms through k_gemm, column
+// sums and activation launches, 1.0 ms so.  Two waves per SIMD (245 VGPRs, the
+// next tile's loads in flight) and one block per CU, which the bases' LDS allows.
+// Needs C = 32, 2 M2 = 16 or 32, k1 = 16 or 32 input channels, n % 32 == 0,
+// n <= 512.  Dynamic LDS: kFnoBwdLds.
+// ---------------------------------------------------------------------------
+enum FnoBwdSrc { kBwdHead = 0, kBwdOut = 1, kBwdDz = 2 };
+
+struct FnoBwdArgs {
+    const float* dout;     // (P, 2)
+    const uint16_t* q16;   // (32, 2)
+    float* dz;             // (P, 32) float32: read (kBwdDz), written (not LIFT, not kBwdHead)
+    const uint16_t* w16;   // (32, 32) W_l, [ci][co]
+    const float* dT;       // (rows, 2 M2, 32)
+    const uint16_t* z;     // (P, 32) z_(l-1)
+    const uint16_t* v;     // (P, 32) v_(l-1), or (LIFT) the input (P, k1)
+    const uint16_t* vL;    // (P, 32): kBwdHead, the projection's input
+    const uint16_t* fyt;   // (n, 2 M2) bf16
+    const uint16_t* gyt;   // (2 M2, n) bf16
+    float* dU;             // (rows, 2 M2, 32)
+    float* part;           // per block: dW (32 x 32), db (32), dQw (64), dqb (2)
+    int64_t rows;
+    int rpw;               // rows per wave
+    int n;
+};
+
+constexpr int kFnoBwdWaves = 8;
+constexpr int kFnoBwdPart = 32 * 32 + 32 + 64 + 2;
+constexpr int kFnoBwdTs = 40;   // bf16 per channel row of a transposed 32-pixel tile
+__host__ __device__ constexpr int fno_fyt_stride(int m2x2) { return m2x2 + 8; }
+// Fy^T and Gy^T, and per wave two transposed tiles; at least the block's
+// partial sums, which reuse it at the end
+__host__ __device__ constexpr size_t kFnoBwdLds(int n, int m2x2) {
+    const size_t a = 2 * ((size_t)n * fno_fyt_stride(m2x2) + (size_t)m2x2 * (n + 8)) +
+                     (size_t)kFnoBwdWaves * 2 * 32 * kFnoBwdTs * 2;
+    const size_t b = (size_t)kFnoBwdWaves * kFnoBwdPart * 4;
+    return a > b ? a : b;
+}
+
+template <int K2F, int SRC, bool LIFT, int K1F>
+__global__ __launch_bounds__(64 * kFnoBwdWaves, 2) void k_fno_bwd_rows(FnoBwdArgs a) {
+    constexpr int m2x2 = 16 * K2F, k1 = 16 * K1F, fs = fno_fyt_stride(m2x2);
+    constexpr bool HEAD = SRC == kBwdHead;
+    static_assert(!(HEAD && LIFT), "the head has a layer below its input");
+    extern __shared__ __align__(16) uint16_t bwd_lds[];
+    __shared__ float lds_q[64];
+    const int n = a.n, gs = n + 8;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l32 = lane & 31, h = lane >> 5;
+    uint16_t* fyt = bwd_lds;                    // [y][m]
+    uint16_t* gyt = fyt + n * fs;               // [m][y]
+    uint16_t* zT = gyt + m2x2 * gs + w * 2 * 32 * kFnoBwdTs;   // [c][y] of the tile's dz
+    uint16_t* vT = zT + 32 * kFnoBwdTs;                        // [c][y] of the tile's v
+    // the bases, 8 bf16 at a time
+    if constexpr (!HEAD)
+        for (int i = threadIdx.x; i < n * m2x2 / 8; i += 64 * kFnoBwdWaves) {
+            const int y = i / (m2x2 / 8), m = i % (m2x2 / 8);
+            *(uint4*)(fyt + y * fs + 8 * m) = *(const uint4*)(a.fyt + 8 * (int64_t)i);
+        }
+    if constexpr (!LIFT)
+        for (int i = threadIdx.x; i < m2x2 * n / 8; i += 64 * kFnoBwdWaves) {
+            const int m = i / (n / 8), y = i % (n / 8);
+            *(uint4*)(gyt + m * gs + 8 * y) = *(const uint4*)(a.gyt + 8 * (int64_t)i);
+        }
+    if (SRC != kBwdDz && threadIdx.x < 64) lds_q[threadIdx.x] = bf16_to_f32(a.q16[threadIdx.x]);
+    __syncthreads();
+
+    // W_l: A(row ci, k co), 8 consecutive co per lane
+    bf16x8_t wf[2];
+    if constexpr (!HEAD) {
+#pragma unroll
+        for (int f = 0; f < 2; ++f) wf[f] = *(const bf16x8_t*)(a.w16 + l32 * 32 + 16 * f + 8 * h);
+    }
+    f32x16_t accW = {};
+    float db[16], dq[HEAD ? 32 : 1], dqb0 = 0.f, dqb1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) db[i] = 0.f;
+#pragma unroll
+    for (int i = 0; i < (HEAD ? 32 : 1); ++i) dq[i] = 0.f;
+
+    // one tile's loads
+    struct Tile {
+        float4 dz[SRC == kBwdDz ? 4 : 1];
+        float2 dout;
+        uint2 z[4], v[4], vL[HEAD ? 4 : 1];
+    };
+    auto load = [&](int64_t row, int y0, Tile& t) __attribute__((always_inline)) {
+        const int64_t pix = row * n + y0 + l32;
+        if constexpr (SRC == kBwdDz) {
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const float4* p = (const float4*)(a.dz + pix * 32 + 16 * f + 8 * h);
+                t.dz[2 * f] = p[0];
+                t.dz[2 * f + 1] = p[1];
+            }
+        } else {
+            t.dout = *(const float2*)(a.dout + pix * 2);
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int c0 = 8 * g + 4 * h;
+            if constexpr (!HEAD && !LIFT) t.z[g] = *(const uint2*)(a.z + pix * 32 + c0);
+            if (8 * g < (LIFT ? k1 : 32))
+                t.v[g] = *(const uint2*)(a.v + pix * (LIFT ? k1 : 32) + c0);
+            if constexpr (HEAD) t.vL[g] = *(const uint2*)(a.vL + pix * 32 + c0);
+        }
+    };
+    auto bits = [](const uint2& q, int j) {
+        const uint32_t word = j < 2 ? q.x : q.y;
+        return (uint16_t)((j & 1) ? word >> 16 : word);
+    };
+    const int64_t r_beg = ((int64_t)blockIdx.x * kFnoBwdWaves + w) * a.rpw;
+    const int64_t r_end = r_beg + a.rpw < a.rows ? r_beg + a.rpw : a.rows;
+    if (r_beg < r_end) {
+        Tile cur, nxt;
+        load(r_beg, 0, cur);
+        for (int64_t row = r_beg; row < r_end; ++row) {
+            // dT_l of this row: A(row c, k m), 8 consecutive m per lane
+            bf16x8_t tf[K2F];
+            if constexpr (!HEAD) {
+                const float* dt = a.dT + row * m2x2 * 32 + l32;
+#pragma unroll
+                for (int f = 0; f < K2F; ++f) {
+                    uint32_t q[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int m = 16 * f + 8 * h + 2 * j;
+                        q[j] = f32x2_to_bf16x2(dt[m * 32], dt[(m + 1) * 32]);
+                    }
+                    tf[f] = __builtin_bit_cast(bf16x8_t, q);
+                }
+            }
+            f32x16_t accU = {};
+            for (int y0 = 0; y0 < n; y0 += 32) {
+                // the next tile: of this row, or the next row's first (the last
+                // one of the wave reads itself again)
+                const bool more = y0 + 32 < n;
+                load(more || row + 1 >= r_end ? row : row + 1,
+                     more ? y0 + 32 : (row + 1 < r_end ? 0 : y0), nxt);
+                const int64_t pix = row * n + y0 + l32;
+                // dz of this tile in the result layout: channels 8 g + 4 h + j
+                float dz[16];
+                float d0 = 0.f, d1 = 0.f;
+                if constexpr (SRC != kBwdDz) {
+                    d0 = bf16_to_f32(f32_to_bf16(cur.dout.x));
+                    d1 = bf16_to_f32(f32_to_bf16(cur.dout.y));
+                }
+                if constexpr (HEAD) {
+                    dqb0 += cur.dout.x;
+                    dqb1 += cur.dout.y;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const int c = 8 * (i >> 2) + 4 * h + (i & 3);
+                        dz[i] = fmaf(d1, lds_q[2 * c + 1], d0 * lds_q[2 * c]);
+                        const float vv = bf16_to_f32(bits(cur.vL[i >> 2], i & 3));
+                        dq[2 * i] = fmaf(vv, d0, dq[2 * i]);
+                        dq[2 * i + 1] = fmaf(vv, d1, dq[2 * i + 1]);
+                    }
+                } else {
+                    f32x16_t acc = {};
+#pragma unroll
+                    for (int f = 0; f < 2; ++f) {
+                        // dz_l: B(k co, col y), 8 consecutive co per lane
+                        float s[8];
+                        if constexpr (SRC == kBwdDz) {
+                            const float4 p = cur.dz[2 * f], q = cur.dz[2 * f + 1];
+                            s[0] = p.x; s[1] = p.y; s[2] = p.z; s[3] = p.w;
+                            s[4] = q.x; s[5] = q.y; s[6] = q.z; s[7] = q.w;
+                        } else {
+#pragma unroll
+                            for (int j = 0; j < 8; ++j) {
+                                const int c = 16 * f + 8 * h + j;
+                                s[j] = fmaf(d1, lds_q[2 * c + 1], d0 * lds_q[2 * c]);
+                            }
+                        }
+                        uint32_t q[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) q[j] = f32x2_to_bf16x2(s[2 * j], s[2 * j + 1]);
+                        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            wf[f], __builtin_bit_cast(bf16x8_t, q), acc, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int f = 0; f < K2F; ++f) {
+                        const bf16x8_t fb =
+                            *(const bf16x8_t*)(fyt + (y0 + l32) * fs + 16 * f + 8 * h);
+                        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tf[f], fb, acc, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        dz[i] = acc[i];
+                        if constexpr (!LIFT)
+                            dz[i] *= gelu_grad(bf16_to_f32(bits(cur.z[i >> 2], i & 3)));
+                    }
+                }
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int c0 = 8 * g + 4 * h;
+                    if constexpr (!HEAD && !LIFT)
+                        *(float4*)(a.dz + pix * 32 + c0) =
+                            make_float4(dz[4 * g], dz[4 * g + 1], dz[4 * g + 2], dz[4 * g + 3]);
+                    const uint2 zb = make_uint2(f32x2_to_bf16x2(dz[4 * g], dz[4 * g + 1]),
+                                                f32x2_to_bf16x2(dz[4 * g + 2], dz[4 * g + 3]));
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        db[4 * g + j] += dz[4 * g + j];
+                        zT[(c0 + j) * kFnoBwdTs + l32] = bits(zb, j);
+                        if (8 * g < (LIFT ? k1 : 32)) vT[(c0 + j) * kFnoBwdTs + l32] = bits(cur.v[g], j);
+                    }
+                }
+                // the tile's transposes are this wave's own: its LDS operations
+                // complete in order, the fence keeps the compiler's order
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int f = 0; f < 2; ++f) {
+                    const bf16x8_t zf = *(const bf16x8_t*)(zT + l32 * kFnoBwdTs + 16 * f + 8 * h);
+                    // rows k1 .. 31 of the input's tile are never written: masked
+                    bf16x8_t vf = *(const bf16x8_t*)(vT + l32 * kFnoBwdTs + 16 * f + 8 * h);
+                    if (LIFT && k1 < 32 && l32 >= k1) vf = bf16x8_t{};
+                    accW = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, zf, accW, 0, 0, 0);
+                    if constexpr (!LIFT) {
+                        bf16x8_t gb = *(const bf16x8_t*)(gyt + (l32 < m2x2 ? l32 : 0) * gs + y0 +
+                                                         16 * f + 8 * h);
+                        accU = __builtin_amdgcn_mfma_f32_32x32x16_bf16(zf, gb, accU, 0, 0, 0);
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                cur = nxt;
+            }
+            if constexpr (!LIFT) {
+                // D(row c, col m): lane m holds channels 8 g + 4 h + 0..3
+                if (l32 < m2x2) {
+                    float* du = a.dU + (row * m2x2 + l32) * 32;
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        *(float4*)(du + 8 * g + 4 * h) = make_float4(
+                            accU[4 * g], accU[4 * g + 1], accU[4 * g + 2], accU[4 * g + 3]);
+                }
+            }
+        }
+    }
+    // per-wave partial sums to LDS (over the bases, which every wave is done
+    // with), added in wave order
+    __syncthreads();
+    float* mine = (float*)bwd_lds + w * kFnoBwdPart;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int c = 8 * (i >> 2) + 4 * h + (i & 3);
+        mine[c * 32 + l32] = accW[i];   // dW(ci = c, co = l32)
+        float s = db[i];
+#pragma unroll
+        for (int d = 1; d < 32; d <<= 1) s += __shfl_xor(s, d);
+        if (l32 == 0) mine[1024 + c] = s;
+        if constexpr (HEAD) {
+            float q0 = dq[2 * i], q1 = dq[2 * i + 1];
+#pragma unroll
+            for (int d = 1; d < 32; d <<= 1) {
+                q0 += __shfl_xor(q0, d);
+                q1 += __shfl_xor(q1, d);
+            }
+            if (l32 == 0) {
+                mine[1056 + 2 * c] = q0;
+                mine[1056 + 2 * c + 1] = q1;
+            }
+        }
+    }
+    if constexpr (HEAD) {
+#pragma unroll
+        for (int d = 1; d < 32; d <<= 1) {
+            dqb0 += __shfl_xor(dqb0, d);
+            dqb1 += __shfl_xor(dqb1, d);
+        }
+        if (lane == 0) {   // both halves hold the same pixels: one counts
+            mine[1120] = dqb0;
+            mine[1121] = dqb1;
+        }
+    }
+    __syncthreads();
+    const int count = HEAD ? kFnoBwdPart : 1056;
+    float* out = a.part + (int64_t)blockIdx.x * kFnoBwdPart;
+    for (int i = threadIdx.x; i < count; i += 64 * kFnoBwdWaves) {
+        float s = 0.f;
+        for (int q = 0; q < kFnoBwdWaves; ++q) s += ((float*)bwd_lds)[q * kFnoBwdPart + i];
+        out[i] = s;
+    }
+}
+
+// The blocks' partial sums added up, all of a launch's gradients at once:
+// out[j] = sum over p < np of part[p kFnoBwdPart + j], written to the gradient
+// the range of j belongs to.  Eight outputs per block, each summed by 32 threads
+// over every 32nd partial and then in order.  (A launch per gradient with eight
+// threads per output: 12 x 11.5 us of a training step.)
+struct FnoGradDst {
+    float *w, *b, *qw, *qb;   // dW (n_w), db (32), dQw (64), dqb (2); qw null: only the first two
+    int n_w;                  // of the 32 x 32 partial block
+};
+__global__ __launch_bounds__(256) void k_part_sum(const float* __restrict__ part, int np,
+                                                  FnoGradDst d) {
+    __shared__ float red[32][9];
+    const int e = threadIdx.x & 7, q = threadIdx.x >> 3;
+    const int j = blockIdx.x * 8 + e;
+    const int end = d.qw ? kFnoBwdPart : 1056;
+    float s = 0.f;
+    if (j < end)
+        for (int p = q; p < np; p += 32) s += part[(int64_t)p * kFnoBwdPart + j];
+    red[q][e] = s;
+    __syncthreads();
+    if (q != 0 || j >= end) return;
+    float t = 0.f;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) t += red[k][e];
+    if (j < 1024) {
+        if (j < d.n_w) d.w[j] = t;
+    } else if (j < 1056) d.b[j - 1024] = t;
+    else if (j < 1120) d.qw[j - 1056] = t;
+    else d.qb[j - 1120] = t;
+}
+
+// dOb[b] (m, nc) = A (m, k) dU[b] (k, nc), A = Gx^T in bf16 rows of k, dU
+// float32 (rounded to bf16 as it is read), m <= 64.  One block per (image, 32
+// columns); the four waves sum a quarter of k each, and their partial tiles are
+// added in LDS.  grid: batch * nc / 32.
+__global__ __launch_bounds__(256) void k_fno_xred(const uint16_t* __restrict__ A,
+                                                  const float* __restrict__ dU,
+                                                  float* __restrict__ out, int m, int k, int nc) {
+    __shared__ float red[4][2][32 * 33];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l32 = lane & 31, h = lane >> 5;
+    const int slabs = nc / 32;
+    const int64_t b = blockIdx.x / slabs;
+    const int c0 = (blockIdx.x % slabs) * 32;
+    const int kq = k / 4;   // a multiple of 16
+    const float* src = dU + b * (int64_t)k * nc + c0 + l32;
+    const uint16_t* ap[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        ap[i] = A + (int64_t)(32 * i + l32 < m ? 32 * i + l32 : 0) * k + 8 * h;
+    f32x16_t acc[2] = {};
+    for (int x0 = w * kq; x0 < (w + 1) * kq; x0 += 64) {
+        // up to four k-steps of 16, all loads first
+        float bv[4][8];
+        bf16x8_t fa[4][2];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int xs = x0 + 16 * s < (w + 1) * kq ? x0 + 16 * s : x0;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) bv[s][r] = src[(int64_t)(xs + 8 * h + r) * nc];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) fa[s][i] = *(const bf16x8_t*)(ap[i] + xs);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if (x0 + 16 * s >= (w + 1) * kq) break;
+            uint32_t q[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) q[r] = f32x2_to_bf16x2(bv[s][2 * r], bv[s][2 * r + 1]);
+            const bf16x8_t fb = __builtin_bit_cast(bf16x8_t, q);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s][i], fb, acc[i], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+            red[w][i][(8 * (v >> 2) + 4 * h + (v & 3)) * 33 + l32] = acc[i][v];
+    __syncthreads();
+    float* o = out + b * (int64_t)m * nc + c0;
+    for (int e = threadIdx.x; e < m * 32; e += 256) {
+        const int row = e >> 5, c = e & 31;
+        float s = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s += red[q][row >> 5][(row & 31) * 33 + c];
+        o[(int64_t)row * nc + c] = s;
+    }
+}
+
+// dT[b] (n, nc) = A (n, k) dPQ[b] (k, nc), A = Fx2^T in bf16 rows of k, dPQ
+// float32 (rounded to bf16), k <= 64.  One wave per 32 x 32 tile, four tiles of
+// adjacent columns per block.  grid: batch * (n / 32) * (nc / 128).
+__global__ __launch_bounds__(256) void k_fno_xexp(const uint16_t* __restrict__ A,
+                                                  const float* __restrict__ dPQ,
+                                                  float* __restrict__ out, int n, int k, int nc) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l32 = lane & 31, h = lane >> 5;
+    const int slabs = nc / 128, rt = n / 32;
+    const int64_t b = blockIdx.x / (slabs * rt);
+    const int rem = (int)(blockIdx.x % (slabs * rt));
+    const int r0 = (rem / slabs) * 32, c0 = (rem % slabs) * 128 + 32 * w;
+    const float* src = dPQ + b * (int64_t)k * nc + c0 + l32;
+    f32x16_t acc = {};
+    float bv[4][8];
+    bf16x8_t fa[4];
+    const int steps = k >> 4;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const int sc = s < steps ? s : 0;
+        fa[s] = *(const bf16x8_t*)(A + (int64_t)(r0 + l32) * k + 16 * sc + 8 * h);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) bv[s][r] = src[(int64_t)(16 * sc + 8 * h + r) * nc];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        if (s >= steps) break;
+        uint32_t q[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) q[r] = f32x2_to_bf16x2(bv[s][2 * r], bv[s][2 * r + 1]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s], __builtin_bit_cast(bf16x8_t, q), acc,
+                                                      0, 0, 0);
+    }
+    float* o = out + (b * n + r0) * (int64_t)nc + c0 + l32;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[(int64_t)(8 * (v >> 2) + 4 * h + (v & 3)) * nc] = acc[v];
+}
+
 // dz = dv * gelu'(z) (act = 1) or dv (act = 0); z bf16, dv / dz float32
 __global__ void k_fno_act_bwd(const float* __restrict__ dv, const uint16_t* __restrict__ z,
                               float* __restrict__ dz, int64_t n, int act) {
