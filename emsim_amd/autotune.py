@@ -26,8 +26,9 @@ KNOBS: Dict[str, Tuple[int, ...]] = {
     "row_items_per_block": (0, 1, 2, 4, 8, 16),
     "col_tiles_per_block": (0, 1, 2, 4, 8),
     # column-transform tile of the propagator pass (256, 512, 1024 points):
-    # 0 = 8 values per thread, 8 columns per block; 1 = half the columns per
-    # block; 2 = 16 values per thread (two radix-8 butterflies per pass)
+    # 0 = 8 values per thread, columns per block by the launch's size; 1 = half
+    # the full tile's columns per block; 2 = 16 values per thread (two radix-8
+    # butterflies per pass)
     "col_shape": (0, 1, 2),
 }
 

@@ -480,18 +480,42 @@ int launch_col_mul_shape(float2* data, int ld, int ncols, int64_t img_stride, in
     return EMSIM_HIP_OK;
 }
 
-// The propagator and last-slice passes of the fused path take the tuned tile
-// shape (emsim_hip_tuning_set("col_shape")) at the lengths that have them.
+// Full-width column tiles a launch over n_img images has (ColDead's skipped
+// tiles left out).
+template <int N>
+int64_t full_col_tiles(int ncols, int n_img, const ColDead& cd) {
+    constexpr int C = ColCfg<N>::C;
+    int64_t per = ceil_div(ncols, C);
+    if (cd.skip_tiles && cd.lo <= cd.hi)
+        per -= std::max<int64_t>((cd.hi + 1) / C - ceil_div(cd.lo, C), 0);
+    return per * n_img;
+}
+
+// The propagator and last-slice passes take the tuned tile shape
+// (emsim_hip_tuning_set("col_shape")) at the lengths that have one; otherwise
+// col_shape_for decides.  The shapes give the same values: each transform's
+// butterflies are the same whichever threads run them.
 template <int N, class Mul>
 int launch_col_mul_impl(float2* data, int ld, int ncols, int64_t img_stride, int n_img, Mul mul,
                         const float2* tw, hipStream_t s, ColDead cd = ColDead{},
                         bool tuned = false) {
-    if constexpr (col_shapes(N)) {
-        if (tuned && g_col_shape == 1)
+    constexpr bool kTunable = col_shapes(N);
+    const int shape = kTunable && tuned && g_col_shape > 0
+                          ? g_col_shape
+                          : col_shape_for<N>(full_col_tiles<N>(ncols, n_img, cd));
+    if constexpr (kTunable || N == 128) {
+        if (shape == 1)
             return launch_col_mul_shape<N, Mul, 1>(data, ld, ncols, img_stride, n_img, mul, tw, s,
                                                    cd);
-        if (tuned && g_col_shape == 2)
+    }
+    if constexpr (kTunable) {
+        if (shape == 2)
             return launch_col_mul_shape<N, Mul, 2>(data, ld, ncols, img_stride, n_img, mul, tw, s,
+                                                   cd);
+    }
+    if constexpr (N == 128 || N == 256) {
+        if (shape == 3)
+            return launch_col_mul_shape<N, Mul, 3>(data, ld, ncols, img_stride, n_img, mul, tw, s,
                                                    cd);
     }
     return launch_col_mul_shape<N, Mul, 0>(data, ld, ncols, img_stride, n_img, mul, tw, s, cd);

@@ -126,11 +126,12 @@ struct RowCfg {
 #ifndef EMSIM_COL_MIN_WAVES
 #define EMSIM_COL_MIN_WAVES 1
 #endif
-// SHAPE selects the tile shape (0: the built-in rule; the others are the
-// alternatives the launch-shape autotuner may pick, see kColShapes):
-//   1: EPT 8, half the columns per block (smaller blocks, more of them per CU)
+// SHAPE selects the tile shape (0: full tiles; col_shape_for picks among 0, 1
+// and 3 by the launch's size, and the launch-shape autotuner may fix 1 or 2):
+//   1: half the columns per block (smaller blocks, more of them)
 //   2: EPT 16 (two radix-8 butterflies per thread and pass, half the threads
 //      per column, the same columns per block)
+//   3: a quarter of the columns per block
 template <int N, int SHAPE = 0>
 struct ColCfg {
     static constexpr int EPT0 = (N / EMSIM_COL_EPT) > 256 ? N / 256
@@ -144,11 +145,30 @@ struct ColCfg {
     static constexpr int CMAX_L = (96 * 1024) / (8 * STRIDE);
     static constexpr int CMAX = CMAX_T < CMAX_L ? CMAX_T : CMAX_L;
     static constexpr int C0 = CMAX < 1 ? 1 : (CMAX < 16 ? CMAX : 16);
-    static constexpr int C = SHAPE == 1 ? (C0 > 1 ? C0 / 2 : 1) : C0;
+    static constexpr int C1 = SHAPE == 1 ? C0 / 2 : (SHAPE == 3 ? C0 / 4 : C0);
+    static constexpr int C = C1 < 1 ? 1 : C1;
     static constexpr int BLOCK = T * C;
 };
-// lengths with alternative column-tile shapes (the others use shape 0)
+// lengths whose tile shape the autotuner may fix (the others use the rule)
 constexpr bool col_shapes(int n) { return n == 256 || n == 512 || n == 1024; }
+// Tile shape of a launch of `tiles` full-width tiles.  A few tiles run on as
+// many CUs, each with all of a block's waves to issue, while the rest idle:
+// narrower tiles spread the same columns over more CUs and shorten the pass
+// to about one wave's own chain of loads and transforms.  The price is narrower
+// segments of the wave's rows -- below 64 bytes the CUs of several XCDs
+// fetch each line -- so 512-point columns (8 to a tile) are only halved, and
+// only where one image is the batch.  Measured, us of a whole run per slice
+// (45 or 30 slices), full / half / quarter tiles: one 256^2 image 12.8 / 11.7 /
+// 11.0, four 16.1 / 14.9 / 14.6, eight (86 tiles) 20.2 / 18.9 / 19.6, sixteen
+// (172 tiles) 29.3 / 29.3 / 29.7; one 128^2 image 11.3 / 10.6 / 10.4, sixteen
+// (96 tiles) 15.6 / 14.8 / 15.2; one 512^2 image (43 tiles) 15.8 / 15.1 /
+// 15.8, two (86 tiles) 16.6 / 17.1 / 20.6 through given potentials.
+template <int N>
+constexpr int col_shape_for(int64_t tiles) {
+    if (N == 128 || N == 256) return tiles <= 48 ? 3 : (tiles <= 128 ? 1 : 0);
+    if (N == 512) return tiles <= 48 ? 1 : 0;
+    return 0;
+}
 
 // Index of this thread's transform within the block; wave-uniform when a
 // transform spans whole waves, so it lives in a scalar register.
@@ -405,9 +425,6 @@ __global__ __launch_bounds__((ColCfg<N, SHAPE>::BLOCK), (col_min_waves<N, SHAPE>
     float* re2 = lds_re2 + (DB ? c * Cfg::STRIDE : 0);
     float* im2 = lds_im2 + (DB ? c * Cfg::STRIDE : 0);
     if (n_tiles <= 0) return;
-    mul.prepare(lds_px, threadIdx.x, Cfg::BLOCK);
-    if constexpr (Mul::kTable) __syncthreads();
-
     int run_start, run_count, parity;
     col_run(blockIdx.x, sched, run_start, run_count, parity);
     // Tile r of this block.  Its loads are never behind a branch: a tile
@@ -417,11 +434,12 @@ __global__ __launch_bounds__((ColCfg<N, SHAPE>::BLOCK), (col_min_waves<N, SHAPE>
     // compiler wait for every load outstanding -- the next tile's included --
     // before the first use of this tile's values.  Tile indices are 32-bit
     // (the launch keeps n_tiles below 2^31).
-    auto tile_at = [&](int r, int& col, bool& ok) __attribute__((always_inline)) -> float2* {
+    auto tile_at = [&](int r, uint32_t& img, int& col,
+                       bool& ok) __attribute__((always_inline)) -> float2* {
         const uint32_t g0 = (uint32_t)(2 * (run_start + r) + parity);
         const bool tile_ok = g0 < (uint32_t)n_tiles;
         const uint32_t g = tile_ok ? g0 : (uint32_t)n_tiles - 1u;
-        const uint32_t img = g / (uint32_t)dcols.live_per_img;
+        img = g / (uint32_t)dcols.live_per_img;
         col = dcols.tile((int)(g - img * (uint32_t)dcols.live_per_img)) * Cfg::C + c;
         ok = tile_ok && col < ncols;
         return data + (int64_t)img * img_stride + (col < ncols ? col : ncols - 1);
@@ -429,19 +447,29 @@ __global__ __launch_bounds__((ColCfg<N, SHAPE>::BLOCK), (col_min_waves<N, SHAPE>
     TwCache<N, EPT> twc;
     twc.load(tw, t);
     float2 cur[EPT], nxt[EPT];
+    uint32_t img;
     int col;
     bool ok;
-    float2* base = tile_at(0, col, ok);
+    float2* base = tile_at(0, img, col, ok);
 #pragma unroll
     for (int m = 0; m < EPT; ++m) cur[m] = base[(int64_t)(t + m * Cfg::T) * ld];
+    // the image's rounding rest (below), loaded with the tile: behind the
+    // column-0 branch it would be a round trip of its own in those tiles
+    const float2* rests = carry ? carry : data;
+    float2 rest_in = rests[carry ? img : 0u];
+    // the row table while the first tile's loads are in flight
+    mul.prepare(lds_px, threadIdx.x, Cfg::BLOCK);
+    if constexpr (Mul::kTable) __syncthreads();
     twc.fence();
     for (int r = 0; r < run_count; ++r) {
         // the next tile (the last one reloads itself, so no branch)
+        uint32_t img_n;
         int col_n;
         bool ok_n;
-        float2* base_n = tile_at(r + 1 < run_count ? r + 1 : r, col_n, ok_n);
+        float2* base_n = tile_at(r + 1 < run_count ? r + 1 : r, img_n, col_n, ok_n);
 #pragma unroll
         for (int m = 0; m < EPT; ++m) nxt[m] = base_n[(int64_t)(t + m * Cfg::T) * ld];
+        const float2 rest_n = rests[carry ? img_n : 0u];
         // a dead column is zero after the propagator whatever it held
         const bool dead = dcols.dead(col);
 #pragma unroll
@@ -457,15 +485,10 @@ __global__ __launch_bounds__((ColCfg<N, SHAPE>::BLOCK), (col_min_waves<N, SHAPE>
         // mean / largest image error 1.15e-6 / 2.0e-6 -> 1.01e-6 / 1.2e-6;
         // 0.2 % of the time of 64 images of 512^2.
         const bool dc = t == 0 && col == 0 && ok;
-        float2 rest = make_float2(0.f, 0.f);
-        float2* slot = nullptr;
-        if (dc && carry) {
-            slot = carry + (base - data) / img_stride;
-            if (!carry_first) rest = *slot;
-        }
+        float2 rest = carry && !carry_first ? rest_in : make_float2(0.f, 0.f);
         if constexpr (DB) fft_n_db<N, EPT, false>(cur, re, im, re2, im2, t, twc, dc ? &rest : nullptr);
         else fft_n<N, EPT, false>(cur, re, im, t, twc, dc ? &rest : nullptr);
-        if (slot) *slot = rest;
+        if (dc && carry) carry[img] = rest;
 #pragma unroll
         for (int m = 0; m < EPT; ++m) cur[m] = mul.apply(cur[m], t + m * Cfg::T, col, lds_px, py);
         if constexpr (DB) fft_n_db<N, EPT, true>(cur, re, im, re2, im2, t, twc);
@@ -476,7 +499,9 @@ __global__ __launch_bounds__((ColCfg<N, SHAPE>::BLOCK), (col_min_waves<N, SHAPE>
         }
 #pragma unroll
         for (int m = 0; m < EPT; ++m) cur[m] = nxt[m];
+        rest_in = rest_n;
         base = base_n;
+        img = img_n;
         col = col_n;
         ok = ok_n;
     }

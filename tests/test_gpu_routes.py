@@ -75,3 +75,24 @@ def test_rectangular_grid_does_not_depend_on_the_batch(hip):
     for k in range(3):
         assert torch.equal(run(square.upload([prepared[k]]))[0], many[k])
     assert np.isfinite(many.cpu().numpy()).all()
+
+
+# (n1, n2, waves): the column pass takes quarter, half or full tiles by the
+# number of full tiles (bounds 48 and 128; 512 rows: half up to 48).  n2 = 8 is
+# narrower than a tile; the waves put the batch on one side of a bound and the
+# waves alone on the other.
+@pytest.mark.parametrize("n1,n2,waves", [(128, 8, 49), (128, 8, 129), (128, 512, 9),
+                                         (256, 256, 3), (256, 256, 8), (256, 16, 49),
+                                         (256, 256, 9), (512, 512, 2), (512, 8, 49),
+                                         (512, 64, 7)])
+def test_wave_does_not_depend_on_the_batch(hip, n1, n2, waves):
+    prop = WavePropagator(n1, n2, 1.0, 1.0, 200.0)
+    gen = torch.Generator(device="cuda").manual_seed(n1 + n2 + waves)
+    v = 40 * torch.rand((waves, 3, n1, n2), generator=gen, device="cuda")
+    psi0 = prop.init_wave(20.0, batch=waves)
+    psi = prop.multislice_propagate(psi0, v, 2.0)
+    image = prop.lens_intensity(psi, 1.3, 700.0, 10e-3)
+    for k in {0, waves // 2, waves - 1}:
+        alone = prop.multislice_propagate(psi0[k], v[k], 2.0)
+        assert torch.equal(alone, psi[k])
+        assert torch.equal(prop.lens_intensity(alone, 1.3, 700.0, 10e-3), image[k])
