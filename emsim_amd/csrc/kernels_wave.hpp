@@ -257,6 +257,10 @@ struct OpTransmit {
     int rows_per_img;
     int64_t v_img_stride;
     float factor;
+    // columns [dead_lo, dead_hi] are zero after the propagator: the first
+    // slice stores zeros there, the later ones take them as they are
+    int dead_lo, dead_hi;
+    __device__ __forceinline__ bool dead(int k) const { return k >= dead_lo && k <= dead_hi; }
     struct Regs {
         float2 v[EPT];
         float p[EPT];
@@ -267,8 +271,12 @@ struct OpTransmit {
         const float* vrow = V + img * v_img_stride + (it - img * rows_per_img) * N;
 #pragma unroll
         for (int m = 0; m < EPT; ++m) {
-            r.v[m] = ok ? src[t + m * T] : make_float2(0.f, 0.f);
-            r.p[m] = ok ? vrow[t + m * T] : 0.f;
+            // the dead columns' zeros all from one of them: its line stays in
+            // the L1 while the others' would come from beyond the L2
+            const int k = t + m * T;
+            const int kw = !FIRST && dead(k) ? dead_lo : k;
+            r.v[m] = ok ? src[kw] : make_float2(0.f, 0.f);
+            r.p[m] = ok ? vrow[k] : 0.f;
         }
     }
     template <class TW>
@@ -285,7 +293,11 @@ struct OpTransmit {
         if (ok) {
             float2* dst = out + it * N;
 #pragma unroll
-            for (int m = 0; m < EPT; ++m) dst[t + m * T] = r.v[m];
+            for (int m = 0; m < EPT; ++m) {
+                const int k = t + m * T;
+                if constexpr (FIRST) dst[k] = dead(k) ? make_float2(0.f, 0.f) : r.v[m];
+                else if (!dead(k)) dst[k] = r.v[m];
+            }
         }
     }
 };
