@@ -67,12 +67,10 @@ __device__ __forceinline__ void dft4(float2& a0, float2& a1, float2& a2, float2&
 template <bool INV>
 __device__ __forceinline__ void dft4(float2* a) { dft4<INV>(a[0], a[1], a[2], a[3]); }
 
+// dft8 from its two halves' length-4 transforms (inputs 0, 2, 4, 6 and 1, 3, 5, 7)
 template <bool INV>
-__device__ __forceinline__ void dft8(float2* a) {
-    float2 e0 = a[0], e1 = a[2], e2 = a[4], e3 = a[6];
-    float2 o0 = a[1], o1 = a[3], o2 = a[5], o3 = a[7];
-    dft4<INV>(e0, e1, e2, e3);
-    dft4<INV>(o0, o1, o2, o3);
+__device__ __forceinline__ void dft8_join(float2* a, float2 e0, float2 e1, float2 e2, float2 e3,
+                                          float2 o0, float2 o1, float2 o2, float2 o3) {
     // o1, o3 times e^{-+i pi/4}, e^{-+3i pi/4}: the factor c goes into the last
     // butterflies' multiply-adds
     const float c = 0.707106781186547524f;
@@ -91,6 +89,44 @@ __device__ __forceinline__ void dft8(float2* a) {
     a[2] = cadd(e2, o2); a[6] = csub(e2, o2);
     a[3] = make_float2(fmaf(c, p3.x, e3.x), fmaf(c, p3.y, e3.y));
     a[7] = make_float2(fmaf(-c, p3.x, e3.x), fmaf(-c, p3.y, e3.y));
+}
+
+template <bool INV>
+__device__ __forceinline__ void dft8(float2* a) {
+    float2 e0 = a[0], e1 = a[2], e2 = a[4], e3 = a[6];
+    float2 o0 = a[1], o1 = a[3], o2 = a[5], o3 = a[7];
+    dft4<INV>(e0, e1, e2, e3);
+    dft4<INV>(o0, o1, o2, o3);
+    dft8_join<INV>(a, e0, e1, e2, e3, o0, o1, o2, o3);
+}
+
+// dft4 of (0, x1, x2, 0), and dft8 whose inputs outside 2 .. 5 (kMidHalf) or
+// 3 .. 4 (kMidQuarter) are zero: the same sums with the zeros left out.
+enum { kMidAll = 0, kMidHalf = 1, kMidQuarter = 2 };
+template <bool INV>
+__device__ __forceinline__ void dft4_mid(float2 x1, float2 x2, float2& a0, float2& a1, float2& a2,
+                                         float2& a3) {
+    const float2 t3 = mul_mi<INV>(x1);
+    a0 = cadd(x2, x1);
+    a2 = csub(x2, x1);
+    a1 = csub(t3, x2);
+    a3 = make_float2(-x2.x - t3.x, -x2.y - t3.y);
+}
+template <bool INV>
+__device__ __forceinline__ void dft8_mid(float2* a, int mid) {
+    float2 e0, e1, e2, e3, o0, o1, o2, o3;
+    if (mid == kMidQuarter) {
+        e0 = e2 = a[4];
+        e1 = e3 = make_float2(-a[4].x, -a[4].y);
+        o0 = a[3];
+        o2 = make_float2(-a[3].x, -a[3].y);
+        o1 = mul_mi<INV>(a[3]);
+        o3 = make_float2(-o1.x, -o1.y);
+    } else {
+        dft4_mid<INV>(a[2], a[4], e0, e1, e2, e3);
+        dft4_mid<INV>(a[3], a[5], o0, o1, o2, o3);
+    }
+    dft8_join<INV>(a, e0, e1, e2, e3, o0, o1, o2, o3);
 }
 
 template <int R, bool INV>
@@ -192,10 +228,12 @@ __device__ __forceinline__ float2 tw_get(const TwLds<N>& c, int q, int r, int k)
 // dc (last pass, thread 0 only, null elsewhere): X[0]'s last sum, of R values,
 // in float64, with *dc added to it; *dc receives what its rounding to float32
 // leaves.
+// mid (leading pass): v[m] is zero outside the middle half or quarter of m, the
+// same for the whole wave (kMidAll: anywhere).
 template <int N, int EPT, int R, int Ns, bool INV, class TW, bool SYNC2 = true>
 __device__ __forceinline__ void stockham_pass(float2 (&v)[EPT], float* __restrict__ re,
                                               float* __restrict__ im, int t, const TW& tw,
-                                              float2* dc = nullptr) {
+                                              float2* dc = nullptr, int mid = kMidAll) {
     constexpr int NB = EPT / R;
     constexpr int S = N / EPT;
     constexpr bool LAST = (Ns * R == N);
@@ -222,7 +260,11 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[EPT], float* __restric
             sum = make_float2((float)sx, (float)sy);
             *dc = make_float2((float)(sx - (double)sum.x), (float)(sy - (double)sum.y));
         }
-        dft<R, INV>(a);
+        if (R == 8 && EPT == 8 && Ns == 1 && mid != kMidAll) {
+            if constexpr (R == 8) dft8_mid<INV>(a, mid);
+        } else {
+            dft<R, INV>(a);
+        }
         if (LAST && q == 0 && dc) a[0] = sum;
         if constexpr (LAST) {
 #pragma unroll
@@ -289,14 +331,14 @@ __device__ __forceinline__ void fft_n_db(float2 (&v)[EPT], float* re0, float* im
 // Unnormalised length-N DFT of the values held by the N/EPT threads of one
 // row/column group.  Every thread of the block must call it (it contains
 // block barriers when N > 8).  tw is the twiddle table (const float2*) or
-// this thread's TwCache<N, EPT>.  dc: see stockham_pass.
+// this thread's TwCache<N, EPT>.  dc, mid: see stockham_pass.
 template <int N, int EPT, bool INV, class TW>
 __device__ __forceinline__ void fft_n(float2 (&v)[EPT], float* re, float* im, int t,
-                                      const TW& tw, float2* dc = nullptr) {
+                                      const TW& tw, float2* dc = nullptr, int mid = kMidAll) {
     static_assert(N >= 8 && N <= kTwN && (N & (N - 1)) == 0, "unsupported FFT length");
     static_assert(EPT >= 8 && EPT % 8 == 0 && EPT <= N, "EPT must be a multiple of 8");
     constexpr int R0 = lead_radix(N);
-    stockham_pass<N, EPT, R0, 1, INV>(v, re, im, t, tw, dc);
+    stockham_pass<N, EPT, R0, 1, INV>(v, re, im, t, tw, dc, mid);
     fft_rest<N, EPT, R0, INV>(v, re, im, t, tw, dc);
 }
 

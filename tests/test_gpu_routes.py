@@ -15,6 +15,8 @@ from emsim_amd.backend._device import ptr, stream_handle
 from emsim_amd.backend.slice_builder_hip import MultiSlicesBuilder
 from emsim_amd.backend.wave_propagator_hip import WavePropagator
 from emsim_amd.batch import BatchPipe
+from oracle import emsim_oracle as orc
+from tests._chain import pipe_oracle
 
 pytestmark = pytest.mark.gpu
 ELEMS = [1, 6, 7, 8, 16]
@@ -118,3 +120,25 @@ def test_multislice_equals_slice_by_slice(hip, n1, n2, d2):
     v[1, 1, 3, 3] = float("nan")
     again = prop.multislice_propagate(psi, v, 2.0)
     assert torch.equal(again[0], many[0]) and not torch.isfinite(again[1]).any()
+
+
+# The spectrum pass leaves out the eighths of the rows beyond the middle quarter
+# or half if an element has no atoms there: atoms up to just inside and just
+# beyond those borders, all columns and both transform kinds (leading radix 8 at
+# 64 and 512 rows, 4 at 256, 2 at 128).  The bound is the other sizes' (1e-5).
+@pytest.mark.parametrize("n", [64, 128, 256, 512])
+@pytest.mark.parametrize("eighths,out", [(1, -0.6), (1, 0.6), (2, -0.6), (2, 0.6), (4, -1.6)])
+def test_rows_in_the_middle_of_the_box(hip, n, eighths, out):
+    half = n * eighths / 8 + out
+    rng = np.random.default_rng(n + eighths)
+    count = 60
+    xyz = np.stack([rng.uniform(-3.5, 3.5, count), rng.uniform(-half, half, count),
+                    rng.uniform(-n / 2 + 2, n / 2 - 2, count)], 1).astype(np.float32)
+    xyz[0, 1], xyz[1, 1] = -half, half          # one element spans the range,
+    xyz[2::3, 1] *= 0.1                         # another stays in the middle
+    zs = np.where(np.arange(count) % 3 == 2, 8, 6)
+    mol = emsim_amd.atoms.AtomList(zs, xyz)
+    pipe = BatchPipe(_tem(), 1.0, 2.0, n, 4, [6, 8])
+    image = pipe.run(pipe.upload([pipe.prepare(mol)]))[0].cpu().numpy()
+    _, exact, _, _ = pipe_oracle(mol, _tem(), 2.0, 2.0, (n, n))
+    assert orc.rel_l2(image, exact) < 1e-5
