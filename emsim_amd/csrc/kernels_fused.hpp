@@ -896,8 +896,13 @@ struct OpSlicePassA {
     int rows_per_img;      // n1
     // wave columns [dead_lo, dead_hi] are zero after every pass B (the
     // propagator's mask); the buffer holds zeros there from the start of
-    // the run, and this pass never stores into them, so they are loaded as
-    // they are
+    // the run, and this pass never stores into them, so no load needs a
+    // branch.  From 512 columns on all the zeros are read from one dead column,
+    // whose line stays in the L1, which takes a third of the wave's reads off
+    // the caches behind it (64 of 512^2 x 100 slices 17.76 -> 17.48 ms); at
+    // 256 columns the per-element offsets cost more (64 of 256^2 x 45 slices
+    // 3,311 -> 3,340 us), so they are loaded as they are.
+    static constexpr bool kOneZero = N >= 512;
     int dead_lo, dead_hi;
     __device__ __forceinline__ bool dead(int k) const { return k >= dead_lo && k <= dead_hi; }
     // raw half-spectrum values of the pair's two rows at this thread's k
@@ -917,7 +922,11 @@ struct OpSlicePassA {
                                            float2 (&w)[EPT]) const {
         const float2* src = wave + (pair * 2 + row) * (int64_t)N;
 #pragma unroll
-        for (int m = 0; m < EPT; ++m) w[m] = ok ? src[t + m * T] : make_float2(0.f, 0.f);
+        for (int m = 0; m < EPT; ++m) {
+            const int k = t + m * T;
+            const int kw = kOneZero && dead(k) ? dead_lo : k;
+            w[m] = ok ? src[kw] : make_float2(0.f, 0.f);
+        }
     }
     template <class TW>
     __device__ __forceinline__ void transmit_row(float2 (&w)[EPT], const float (&V)[EPT], int t,
