@@ -1567,8 +1567,8 @@ template <int N>
 int launch_spec_sparse(const uint32_t* row_start, const uint16_t* bucket, const float* sf,
                        const float* sft, float2* Y, int slice0, int n_sc, int n_slices,
                        int n_elems, int H, int ldh, int n2, int bandlimit, int band_r2,
-                       float inv_npix, int batch, const int* order, const float2* tw,
-                       hipStream_t s) {
+                       float inv_npix, int batch, const int* order, const WaterPlanes& wp,
+                       const float2* tw, hipStream_t s) {
     using Cfg = SpecCfg<N>;
     if (H != n2 / 2 + 1 || n2 < 2 || ldh < H + n_elems)
         return fail(EMSIM_HIP_EINVAL, "spectrum: needs H = n2/2 + 1, n2 >= 2, ldh >= H + n_elems");
@@ -1578,9 +1578,30 @@ int launch_spec_sparse(const uint32_t* row_start, const uint16_t* bucket, const 
     if (blocks >= ((int64_t)1 << 31))
         return fail(EMSIM_HIP_EINVAL, "spectrum: %lld blocks, at most 2^31 - 1", (long long)blocks);
     if (!sft) return fail(EMSIM_HIP_EINVAL, "spectrum: no tile-major form-factor table");
-    EMSIM_LAUNCH(N, (k_spec_sparse<N>), dim3((unsigned)blocks), dim3(Cfg::BLOCK), 0, s, row_start,
-                 bucket, sf, sft, Y, slice0, n_sc, n_slices, n_elems, H, ldh, n2, batch, bandlimit,
-                 band_r2, inv_npix, order, tw);
+    if (wp.X)
+        EMSIM_LAUNCH(N, (k_spec_sparse<N, true>), dim3((unsigned)blocks), dim3(Cfg::BLOCK), 0, s,
+                     row_start, bucket, sf, sft, Y, slice0, n_sc, n_slices, n_elems, H, ldh, n2,
+                     batch, bandlimit, band_r2, inv_npix, order, wp, tw);
+    else
+        EMSIM_LAUNCH(N, (k_spec_sparse<N, false>), dim3((unsigned)blocks), dim3(Cfg::BLOCK), 0, s,
+                     row_start, bucket, sf, sft, Y, slice0, n_sc, n_slices, n_elems, H, ldh, n2,
+                     batch, bandlimit, band_r2, inv_npix, order, wp, tw);
+    return EMSIM_HIP_OK;
+}
+
+// Rows dealt out evenly over one round of resident blocks, as in pass A.
+template <int N>
+int launch_water_rows(const WaterRows& a, int n_sc, const float2* tw, hipStream_t s) {
+    static int resident_cache[64];
+    const int64_t resident =
+        resident_blocks(k_water_rows<N>, RowCfg<N>::BLOCK, resident_cache);
+    const int64_t n_rows = (int64_t)n_sc * a.batch * a.n1, groups = ceil_div(n_rows, RowCfg<N>::G);
+    if (groups <= 0) return EMSIM_HIP_OK;
+    int64_t blocks = resident > 0 ? resident : 2048;
+    if (blocks > groups) blocks = groups;
+    const RunSched sched{(int)(groups / blocks), (int)(groups % blocks)};
+    EMSIM_LAUNCH(N, (k_water_rows<N>), dim3((unsigned)blocks), dim3(RowCfg<N>::BLOCK), 0, s, a,
+                 n_rows, sched, tw);
     return EMSIM_HIP_OK;
 }
 
@@ -1665,9 +1686,12 @@ int launch_col_lensprop(float2* data, int ld, int ncols, int64_t img_stride, int
 int spec_sparse(int n, const uint32_t* row_start, const uint16_t* bucket, const float* sf,
                 const float* sft, float2* Y, int slice0, int n_sc, int n_slices, int n_elems,
                 int H, int ldh, int n2, int bandlimit, int band_r2, float inv_npix, int batch,
-                const int* order, const float2* tw, hipStream_t s) {
+                const int* order, const WaterPlanes& wp, const float2* tw, hipStream_t s) {
     EMSIM_DISPATCH(n, launch_spec_sparse, row_start, bucket, sf, sft, Y, slice0, n_sc, n_slices,
-                   n_elems, H, ldh, n2, bandlimit, band_r2, inv_npix, batch, order, tw, s);
+                   n_elems, H, ldh, n2, bandlimit, band_r2, inv_npix, batch, order, wp, tw, s);
+}
+int water_rows(int n, const WaterRows& a, int n_sc, const float2* tw, hipStream_t s) {
+    EMSIM_DISPATCH(n, launch_water_rows, a, n_sc, tw, s);
 }
 int phase_rows(int n, const float2* Y, float2* phase, int n_sc, int batch, int n1, int ldh,
                float factor, float* vout, int slice0, int n_slices, const float2* tw,
@@ -1714,9 +1738,10 @@ bool fused_split(const emsim_hip_slice_builder* b, int batch) {
 // 5,478 / 5,352 / 5,424 us for 32 of 512^2 x 50).
 constexpr int64_t kChunkBytes = (int64_t)192 << 20;
 constexpr int64_t kMinChunk = 8;
-int fused_chunk(const emsim_hip_slice_builder* b, int batch) {
+int fused_chunk(const emsim_hip_slice_builder* b, int batch, bool water) {
     const int64_t rows = (int64_t)batch * b->n1;
-    const int64_t per = rows * (fused_ld(b) + (fused_split(b, batch) ? b->n2 : 0)) *
+    const int64_t per = rows * (fused_ld(b) + (fused_split(b, batch) ? b->n2 : 0) +
+                                (water ? 2 * half_ld(b->H) : 0)) *
                         (int64_t)sizeof(float2);
     const int64_t c = std::max(kChunkBytes / per, kMinChunk);
     return (int)std::min(c, (int64_t)b->n_slices);
@@ -1737,9 +1762,8 @@ struct FusedWorkspace {
     float2* Y;
     float2* wave;
     float2* carry;    // (batch): rounding rests of the waves' means (pass B)
-    // water fill (emsim_hip_simulate_water): dense count planes and half
-    // spectra of one slice of every molecule, per-molecule seeds
-    float* hist;
+    // water fill (emsim_hip_simulate_water): half spectra of the hydrogen and
+    // oxygen rows (chunk, batch, 2, n1, half_ld(H)), per-molecule seeds
     float2* X;
     uint64_t* seeds;
     // molecules given as they come (emsim_hip_simulate_raw): per-atom element
@@ -1761,7 +1785,7 @@ struct WaterFill {
 FusedWorkspace fused_layout(const emsim_hip_slice_builder* b, int batch, int64_t n_atoms,
                             bool own_wave, char* base, bool water = false, bool raw = false) {
     FusedWorkspace w;
-    w.chunk = water ? 1 : fused_chunk(b, batch);
+    w.chunk = fused_chunk(b, batch, water);
     w.n_rows = (int64_t)batch * b->n_slices * b->n_elems * b->n1;
     const int64_t n_scan = w.n_rows + 1;
     const int64_t n_blocks = ceil_div(n_scan, kScanTile);
@@ -1781,7 +1805,7 @@ FusedWorkspace fused_layout(const emsim_hip_slice_builder* b, int batch, int64_t
     w.Y = (float2*)(base + off);
     off += align_up(sizeof(float2) * (size_t)w.chunk * batch * b->n1 * ldh);
     w.phase = nullptr;
-    if (!water && fused_split(b, batch)) {
+    if (fused_split(b, batch)) {
         w.phase = (float2*)(base + off);
         off += align_up(sizeof(float2) * (size_t)w.chunk * batch * b->n1 * b->n2);
     }
@@ -1792,13 +1816,11 @@ FusedWorkspace fused_layout(const emsim_hip_slice_builder* b, int batch, int64_t
     }
     w.carry = (float2*)(base + off);
     off += align_up(sizeof(float2) * (size_t)batch);
-    w.hist = nullptr;
     w.X = nullptr;
     w.seeds = nullptr;
     if (water) {
-        const size_t planes = (size_t)b->n_elems * batch * b->n1;
-        w.hist = (float*)(base + off);   off += align_up(sizeof(float) * planes * b->n2);
-        w.X = (float2*)(base + off);     off += align_up(sizeof(float2) * planes * half_ld(b->H));
+        w.X = (float2*)(base + off);
+        off += align_up(sizeof(float2) * 2 * (size_t)w.chunk * batch * b->n1 * half_ld(b->H));
         w.seeds = (uint64_t*)(base + off); off += align_up(sizeof(uint64_t) * (size_t)batch);
     }
     w.atom_elem = nullptr;
@@ -1949,7 +1971,7 @@ extern "C" int emsim_hip_simulate_water(const emsim_hip_slice_builder* b,
         return fail(EMSIM_HIP_EINVAL, "simulate_water: bad water arguments");
     if ((size_t)b->n_elems * b->n2 * sizeof(float) > 64 * 1024)
         return fail(EMSIM_HIP_EUNSUPPORTED,
-                    "simulate_water: n_elems * n2 <= 16384 (one row of every element in LDS)");
+                    "simulate_water: n_elems * n2 <= 16384");
     std::vector<int64_t> elem_off;
     rc = host_offsets(b, mol_off_host, elem_counts_host, batch, n_atoms, elem_off);
     if (rc) return rc;
@@ -2176,47 +2198,35 @@ int simulate_core(const emsim_hip_slice_builder* b, const emsim_hip_wave_propaga
     for (int sl = 0; sl < b->n_slices; ++sl) {
         const bool last = sl == b->n_slices - 1;
         dead.carry_first = dead_last.carry_first = sl == 0;
-        if (!water.on) {
-            const int sc = sl % ws.chunk;   // plane of this slice in its chunk
-            if (sc == 0) {
-                const int n_sc = std::min(ws.chunk, b->n_slices - sl);
-                rc = spec_sparse(b->n1, ws.row_start, ws.bucket, b->sf, b->sf_tiles, ws.Y, sl,
-                                 n_sc, b->n_slices, b->n_elems, b->H, ldh, b->n2,
-                                 symmetric_bandlimit ? 1 : 0, r * r, inv_npix, batch, order,
-                                 b->tw, s);
-                if (!rc && ws.phase)
-                    rc = phase_rows(b->n2, ws.Y, ws.phase, n_sc, batch, b->n1, ldh, w->factor,
-                                    slices_out, sl, b->n_slices, b->tw, s);
+        const int sc = sl % ws.chunk;   // plane of this slice in its chunk
+        if (sc == 0) {
+            const int n_sc = std::min(ws.chunk, b->n_slices - sl);
+            WaterPlanes wp{nullptr, 0, 0, 0};
+            if (water.on) {
+                wp = WaterPlanes{ws.X, water.idx_h, water.idx_o, half_ld(b->H)};
+                rc = water_rows(b->n2,
+                                WaterRows{ws.row_start, ws.bucket, ws.seeds, ws.X, sl, b->n_slices,
+                                          b->n_elems, b->n1, batch, wp.ldx, water.idx_h,
+                                          water.idx_o, water.lam_o, water.exp_o, water.lam_h,
+                                          water.exp_h},
+                                n_sc, b->tw, s);
                 if (rc) return rc;
             }
-            if (ws.phase)
-                rc = phase_apply(b->n2, sl == 0, ws.phase + sc * batch * npix, wave, rows, psi0,
-                                 dead, b->tw, s);
-            else
-                rc = slice_pass_a(b->n2, sl == 0, ws.Y + (int64_t)sc * rows * ldh, wave, rows / 2,
-                                  ldh, psi0, w->factor, slices_out, sl, b->n_slices, b->n1, dead,
-                                  b->tw, s);
-            if (rc) return rc;
-        } else {
-            // water: dense count planes of this slice (atoms + water), then
-            // the reference-shaped R2C and spectrum column pass; Y = X[0]
-            const int ldx = half_ld(b->H);
-            const size_t lds = sizeof(float) * (size_t)b->n_elems * b->n2;
-            EMSIM_LAUNCH(0, k_dense_slice_rows, dim3((unsigned)(batch * (int64_t)b->n1)),
-                         dim3(256), lds, s, ws.row_start, ws.bucket, sl, b->n_slices,
-                         b->n_elems, b->n1, b->n2, batch, ws.hist, 1, water.idx_h, water.idx_o,
-                         water.lam_o, water.exp_o, water.lam_h, water.exp_h,
-                         (const uint64_t*)ws.seeds);
-            rc = r2c_pairs(b->n2, ws.hist, ws.X, (int64_t)b->n_elems * batch * (b->n1 / 2), b->n1,
-                           batch, batch, 0, ldx, b->tw, s);
-            if (rc) return rc;
-            rc = col_spectrum(b->n1, ws.X, b->sf, b->n_elems, batch, b->H, ldx, b->n2,
-                              symmetric_bandlimit ? 1 : 0, r * r, inv_npix, b->tw, s);
-            if (rc) return rc;
-            rc = slice_pass_a(b->n2, sl == 0, ws.X, wave, rows / 2, ldx, psi0, w->factor,
-                              slices_out, sl, b->n_slices, b->n1, dead, b->tw, s);
+            rc = spec_sparse(b->n1, ws.row_start, ws.bucket, b->sf, b->sf_tiles, ws.Y, sl, n_sc,
+                             b->n_slices, b->n_elems, b->H, ldh, b->n2, symmetric_bandlimit ? 1 : 0,
+                             r * r, inv_npix, batch, order, wp, b->tw, s);
+            if (!rc && ws.phase)
+                rc = phase_rows(b->n2, ws.Y, ws.phase, n_sc, batch, b->n1, ldh, w->factor,
+                                slices_out, sl, b->n_slices, b->tw, s);
             if (rc) return rc;
         }
+        if (ws.phase)
+            rc = phase_apply(b->n2, sl == 0, ws.phase + sc * batch * npix, wave, rows, psi0, dead,
+                             b->tw, s);
+        else
+            rc = slice_pass_a(b->n2, sl == 0, ws.Y + (int64_t)sc * rows * ldh, wave, rows / 2, ldh,
+                              psi0, w->factor, slices_out, sl, b->n_slices, b->n1, dead, b->tw, s);
+        if (rc) return rc;
         if (mode == 0 && last) {
             LensPropMul lp;
             lp.p = prop;

@@ -163,51 +163,6 @@ __global__ __launch_bounds__(kSortRows) void k_csr_sort_rows(int64_t n_rows,
     for (uint32_t i = threadIdx.x; i < hi - lo; i += kSortRows) bucket[lo + i] = lds[i];
 }
 
-// Dense count planes of one slice of every molecule, with the water fill.
-// One block per (molecule b, row x): the nE rows (b, slice, e, x) of the
-// atom buckets are counted into LDS (integer-valued float adds, exact and
-// order-independent), then -- with water -- every voxel y empty for all
-// elements gets Poisson oxygens and hydrogens drawn exactly as k_add_water
-// draws them for voxel v = (slice n1 + x) n2 + y of a (n_slices, n1, n2)
-// histogram with the molecule's seed; the rows are written to
-// hist (n_elems, batch, n1, n2).  Dynamic LDS: n_elems * n2 floats.
-__global__ __launch_bounds__(256) void k_dense_slice_rows(
-    const uint32_t* __restrict__ row_start, const uint16_t* __restrict__ bucket, int slice,
-    int n_slices, int n_elems, int n1, int n2, int batch, float* __restrict__ hist, int water,
-    int idx_h, int idx_o, float lam_o, float exp_o, float lam_h, float exp_h,
-    const uint64_t* __restrict__ seeds) {
-    extern __shared__ float rows[];
-    const int b = (int)(blockIdx.x / (unsigned)n1), x = (int)(blockIdx.x % (unsigned)n1);
-    const int words = n_elems * n2;
-    for (int i = threadIdx.x; i < words; i += blockDim.x) rows[i] = 0.f;
-    __syncthreads();
-    for (int e = 0; e < n_elems; ++e) {
-        const int64_t r = (((int64_t)b * n_slices + slice) * n_elems + e) * n1 + x;
-        const uint32_t beg = row_start[r], end = row_start[r + 1];
-        for (uint32_t k = beg + threadIdx.x; k < end; k += blockDim.x)
-            atomicAdd(&rows[e * n2 + bucket[k]], 1.f);
-    }
-    __syncthreads();
-    if (water) {
-        const uint64_t seed = seeds[b];
-        for (int y = threadIdx.x; y < n2; y += blockDim.x) {
-            bool empty = true;
-            for (int e = 0; e < n_elems; ++e) empty = empty && (rows[e * n2 + y] == 0.f);
-            if (!empty) continue;
-            const uint64_t v = ((uint64_t)slice * (uint64_t)n1 + (uint64_t)x) * (uint64_t)n2 +
-                               (uint64_t)y;
-            const uint64_t key = splitmix64(seed ^ splitmix64(v));
-            rows[idx_o * n2 + y] += poisson_draw(splitmix64(key + 1), exp_o, lam_o);
-            rows[idx_h * n2 + y] += poisson_draw(splitmix64(key + 2), exp_h, lam_h);
-        }
-        __syncthreads();
-    }
-    for (int i = threadIdx.x; i < words; i += blockDim.x) {
-        const int e = i / n2, y = i - e * n2;
-        hist[(((int64_t)e * batch + b) * n1 + x) * n2 + y] = rows[i];
-    }
-}
-
 // Spectrum-pass molecule slots of every slice: slot r of slice s is the
 // molecule with the r-th most atoms in that slice (ties by index).  One
 // block per slice, one thread per molecule (batch <= blockDim.x); a
@@ -230,6 +185,115 @@ __global__ void k_slice_order(const uint32_t* __restrict__ row_start, int n_slic
             rank += (o > c || (o == c && j < i)) ? 1 : 0;
         }
         order[(int64_t)s * batch + rank] = i;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Water rows of slices slice0 .. slice0 + n_sc - 1: the half spectra of the
+// hydrogen and oxygen rows with the water fill, X (n_sc, batch, 2, n1, ldx).
+// Item = row x of a (slice, molecule) plane.  The row's atoms (all elements)
+// mark their voxels in LDS and the hydrogens and oxygens are counted there
+// (integer-valued float adds, exact and order-independent); every voxel y
+// empty of all elements then gets Poisson oxygens and hydrogens drawn as
+// k_add_water draws them for voxel (slice n1 + x) n2 + y of a (n_slices, n1,
+// n2) histogram with the molecule's seed.  Both rows are real, so one complex
+// transform of h + i o gives both spectra; the other elements stay in their
+// buckets for k_spec_sparse.  What bounds it: the 64-bit products of the counter-based
+// draws (VALU), and a row's chain of table, bucket and LDS latencies, hidden by
+// the CU's other waves (16 molecules of 256^2: 6.0 us a slice, where count planes of
+// all elements, 21 MB written and read back, and a transform per pair of rows took 30.5).
+// ---------------------------------------------------------------------------
+struct WaterRows {
+    const uint32_t* row_start;
+    const uint16_t* bucket;
+    const uint64_t* seeds;
+    float2* X;
+    int slice0, n_slices, n_elems, n1, batch, ldx;
+    int idx_h, idx_o;
+    float lam_o, exp_o, lam_h, exp_h;
+};
+template <int N>
+__global__ __launch_bounds__(RowCfg<N>::BLOCK) void k_water_rows(WaterRows a, int64_t n_rows,
+                                                                 RunSched sched,
+                                                                 const float2* __restrict__ tw) {
+    using Cfg = RowCfg<N>;
+    using L = LdsLayout<N>;
+    constexpr int EPT = Cfg::EPT, T = Cfg::T, H = N / 2 + 1;
+    __shared__ float lds_re[Cfg::G * Cfg::WORDS];
+    __shared__ float lds_im[Cfg::G * Cfg::WORDS];
+    __shared__ uint32_t lds_occ[Cfg::G * N];
+    const int gi = row_in_block<T>();
+    const int t = threadIdx.x % T;
+    float* re = lds_re + gi * Cfg::WORDS;   // hydrogens, then the transform's planes
+    float* im = lds_im + gi * Cfg::WORDS;   // oxygens
+    uint32_t* occ = lds_occ + gi * N;
+    int run_start, run_count;
+    sched.run((int)blockIdx.x, run_start, run_count);
+    TwCache<N, EPT> twc;
+    twc.load(tw, t);
+    // lanes per element: a power of two, so that T threads take whole elements
+    int per = T;
+    while (per > 1 && (T / per) < a.n_elems) per >>= 1;
+    for (int r = 0; r < run_count; ++r) {
+        const int64_t it = ((int64_t)run_start + r) * Cfg::G + gi;
+        const bool ok = it < n_rows;
+        const int64_t row = ok ? it : n_rows - 1;
+        const int64_t plane = row / a.n1;               // sc batch + b
+        const int x = (int)(row - plane * a.n1);
+        const int sc = (int)(plane / a.batch), b = (int)(plane - (int64_t)sc * a.batch);
+        const int slice = a.slice0 + sc;
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            re[t + m * T] = 0.f;
+            im[t + m * T] = 0.f;
+            occ[t + m * T] = 0u;
+        }
+        __syncthreads();
+        for (int e = t / per; e < a.n_elems; e += T / per) {
+            const int64_t br = (((int64_t)b * a.n_slices + slice) * a.n_elems + e) * a.n1 + x;
+            const uint32_t end = a.row_start[br + 1];
+            for (uint32_t k = a.row_start[br] + (uint32_t)(t % per); k < end; k += (uint32_t)per) {
+                const int y = a.bucket[k];
+                occ[y] = 1u;
+                if (e == a.idx_h) atomicAdd(&re[y], 1.f);
+                if (e == a.idx_o) atomicAdd(&im[y], 1.f);
+            }
+        }
+        __syncthreads();
+        float2 v[EPT];
+        const uint64_t seed = a.seeds[b];
+        const uint64_t voxel0 = ((uint64_t)slice * (uint64_t)a.n1 + (uint64_t)x) * (uint64_t)N;
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            const int y = t + m * T;
+            v[m] = make_float2(re[y], im[y]);
+            if (occ[y] == 0u) {
+                const uint64_t key = splitmix64(seed ^ splitmix64(voxel0 + (uint64_t)y));
+                v[m].y += poisson_draw(splitmix64(key + 1), a.exp_o, a.lam_o);
+                v[m].x += poisson_draw(splitmix64(key + 2), a.exp_h, a.lam_h);
+            }
+        }
+        __syncthreads();   // the counts are read: the planes are the transform's
+        fft_n<N, EPT, false>(v, re, im, t, twc);
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            const int idx = L::at(t + m * T);
+            re[idx] = v[m].x;
+            im[idx] = v[m].y;
+        }
+        __syncthreads();
+        if (ok) {
+            float2* xh = a.X + ((plane * 2) * a.n1 + x) * (int64_t)a.ldx;
+            float2* xo = xh + (int64_t)a.n1 * a.ldx;
+            for (int k = t; k < H; k += T) {
+                const int ik = L::at(k & (N - 1)), inr = L::at((N - k) & (N - 1));
+                const float zr = re[ik], zi = im[ik];
+                const float wr = re[inr], wi = -im[inr];   // conj Z[N - k]
+                xh[k] = make_float2(0.5f * (zr + wr), 0.5f * (zi + wi));
+                xo[k] = make_float2(0.5f * (zi - wi), -0.5f * (zr - wr));
+            }
+        }
+        __syncthreads();   // the next row's counts overwrite the planes
     }
 }
 
@@ -488,12 +552,19 @@ __device__ __forceinline__ void spec_fft(float2 (&v)[EPT], float* re, float* im,
     else fft_n<N, EPT, INV>(v, re, im, t, tw, nullptr, mid);
 }
 
-template <int N>
+// The water path's two dense elements: their rows' half spectra as k_water_rows
+// writes them (planes 2 p + 0 / 1 of (slice, molecule) plane p).
+struct WaterPlanes {
+    const float2* X;
+    int idx_h, idx_o, ldx;
+};
+
+template <int N, bool WATER>
 __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_SPEC_MIN_WAVES : 1) void k_spec_sparse(
     const uint32_t* __restrict__ row_start, const uint16_t* __restrict__ bucket,
     const float* __restrict__ sf, const float* __restrict__ sft, float2* __restrict__ Y,
     int slice0, int n_sc, int n_slices, int n_elems, int H, int ldh, int n2, int batch,
-    int bandlimit, int band_r2, float inv_npix, const int* __restrict__ order,
+    int bandlimit, int band_r2, float inv_npix, const int* __restrict__ order, WaterPlanes wp,
     const float2* __restrict__ tw) {
     using Cfg = SpecCfg<N>;
     constexpr int EPT = Cfg::EPT;
@@ -655,8 +726,9 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
             e_end = __builtin_amdgcn_readfirstlane(row_start[rbase + (e + 1) * N]);
         }
         const uint32_t n_e = e_end - e_beg;
+        const bool dense = WATER && (e == wp.idx_h || e == wp.idx_o);
         // an element without atoms in this slice adds exactly zero
-        if (n_e == 0) {
+        if (n_e == 0 && !dense) {
             if (packed) {
 #pragma unroll
                 for (int m = 0; m < EPT; ++m)
@@ -673,7 +745,21 @@ __global__ __launch_bounds__(SpecCfg<N>::BLOCK, (N >= 512 && N <= 1024) ? EMSIM_
 #pragma unroll
         for (int m = 0; m < EPT; ++m) fe[m] = f[(int64_t)m * Cfg::T * Cfg::C];
         float2 v[EPT];
-        if (all_lds && n_e <= (uint32_t)kSpecDirect) {
+        if (dense) {
+            // the row transforms are given; columns beyond H read the last one
+            // (their results are not stored)
+            const float2* src = wp.X + (((int64_t)sc * batch + b) * 2 + (e == wp.idx_o ? 1 : 0)) *
+                                           N * wp.ldx;
+            const int cl = col < H ? col : H - 1;
+#pragma unroll
+            for (int m = 0; m < EPT; ++m) v[m] = src[(int64_t)(t + m * Cfg::T) * wp.ldx + cl];
+            if (packed) {   // column 0 + i column n2/2, both real
+#pragma unroll
+                for (int m = 0; m < EPT; ++m)
+                    v[m].y = src[(int64_t)(t + m * Cfg::T) * wp.ldx + half].x;
+            }
+            spec_fft<N, EPT, false, kTwCached>(v, re, im, t, twc, tw);
+        } else if (all_lds && n_e <= (uint32_t)kSpecDirect) {
             // few atoms: their 2-D DFT sum_a w_N^(k x_a) w_n2^(col y_a) directly,
             // cheaper than a column transform (the y factor is the twiddle the
             // row DFT would use, the x factor the transform's table entry)

@@ -202,9 +202,9 @@ int emsim_hip_simulate(const emsim_hip_slice_builder* b, const emsim_hip_wave_pr
  * Poisson(2 voxel_water) hydrogens in the planes of elements idx_o / idx_h.
  * Molecule m draws with seeds_host[m] exactly the values
  * emsim_hip_add_water draws with that seed for the molecule's own
- * (n_slices, n1, n2) histogram.  Slices are formed from dense count planes
- * (the reference's R2C + spectrum pass) rather than the sparse spectrum
- * pass.  Multi-slice builders only; n_elems * n2 <= 16384. */
+ * (n_slices, n1, n2) histogram.  The hydrogen and oxygen rows are counted,
+ * filled and transformed as dense rows, the other elements go through the
+ * sparse spectrum pass.  Multi-slice builders only; n_elems * n2 <= 16384. */
 size_t emsim_hip_simulate_water_workspace_size(const emsim_hip_slice_builder* b, int batch,
                                                int64_t n_atoms, int mode);
 int emsim_hip_simulate_water(const emsim_hip_slice_builder* b, const emsim_hip_wave_propagator* w,

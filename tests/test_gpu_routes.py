@@ -2,7 +2,7 @@
 the spectrum pass (up to a bound of plane memory) and pass A in one kernel or
 two (up to a bound of pixels).  Every choice runs the same operations on the
 same values, so a molecule's result is the same bits in any batch."""
-from ctypes import POINTER, c_int64
+from ctypes import POINTER, c_int64, c_uint64
 
 import numpy as np
 import pytest
@@ -142,3 +142,45 @@ def test_rows_in_the_middle_of_the_box(hip, n, eighths, out):
     image = pipe.run(pipe.upload([pipe.prepare(mol)]))[0].cpu().numpy()
     _, exact, _, _ = pipe_oracle(mol, _tem(), 2.0, 2.0, (n, n))
     assert orc.rel_l2(image, exact) < 1e-5
+
+
+# The water path: hydrogen and oxygen rows from one transform, the others from
+# their buckets.  Rows shorter than a wave and longer than one, more elements than
+# threads per row, both routes of pass A, several launches of the spectrum pass, the
+# packed column of 2048 rows, rectangles.  Potentials against the dense ones of
+# the same counts (the bound is the other sizes', 1e-5).
+@pytest.mark.parametrize("n1,n2,slices,elems,count", [
+    (8, 8, 3, [1, 6, 8], 2), (16, 64, 2, [1, 8], 3), (64, 16, 9, [1, 6, 7, 8, 16], 2),
+    (128, 128, 5, [1, 6, 7, 8, 16], 40), (256, 256, 21, [1, 6, 7, 8, 16], 9),
+    (1024, 32, 2, [1, 6, 8], 1), (512, 1024, 1, [1, 8], 1), (2048, 64, 2, [1, 6, 8], 2)])
+def test_water_potentials_equal_dense_ones(hip, n1, n2, slices, elems, count):
+    dz, d1, d2 = 2.0, 1.0, 1.0
+    builder = MultiSlicesBuilder(elems, slices, n1, n2, dz, d1, d2)
+    prop = WavePropagator(n1, n2, d1, d2, 200.0).backend
+    rng = np.random.default_rng(n1 + n2)
+    counts = rng.integers(0, 60, (count, len(elems))).astype(np.int64)
+    off = np.concatenate([[0], np.cumsum(counts.sum(axis=1))]).astype(np.int64)
+    n_atoms = int(off[-1])
+    half = np.array([slices * dz, n1 * d1, n2 * d2]) / 2
+    coords = torch.from_numpy(rng.uniform(-half, half, (n_atoms, 3)).astype(np.float32)).cuda()
+    seeds = rng.integers(0, 2 ** 62, count).astype(np.uint64)
+    band = 1 if n1 == n2 else 0
+    image = torch.empty((count, n1, n2), device="cuda")
+    v = torch.full((count, slices, n1, n2), -1.0, device="cuda")
+    need = hip_ext.raw("emsim_hip_simulate_water_workspace_size")(builder.backend.h, count,
+                                                                   n_atoms, 0)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    args = (builder.backend.h, prop.h, ptr(coords), n_atoms, off.ctypes.data_as(POINTER(c_int64)),
+            np.ascontiguousarray(counts).ctypes.data_as(POINTER(c_int64)), count, 4.5, 1.3, 700.0,
+            10e-3, band, elems.index(1), elems.index(8),
+            emsim_amd.physics.water_num_dens * d1 * d2 * dz,
+            seeds.ctypes.data_as(POINTER(c_uint64)), ptr(image), ptr(v), 0, ptr(ws))
+    rc = hip_ext.raw("emsim_hip_simulate_water")(*args, need - 1, stream_handle())
+    assert rc == hip_ext.EWORKSPACE
+    hip_ext.call("emsim_hip_simulate_water", *args, need, stream_handle())
+    for b in range(count):
+        hist = builder.backend.bin_atoms(coords[off[b]:off[b + 1]], counts[b])
+        hist = builder.add_water(hist, seed=int(seeds[b]))
+        ref = builder.backend.make_slices(hist, bool(band))
+        assert float((v[b] - ref).norm() / ref.norm()) < 1e-5, b
+    assert torch.isfinite(image).all()
