@@ -131,18 +131,37 @@ __device__ __forceinline__ void sort_row(uint16_t* a, uint32_t len) {
     }
 }
 
+// Orders a wave's LDS accesses before and after it (they execute in order; this
+// keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Sort every bucket row's y bins ascending, which fixes the order of the
 // float row sums.  One block per kSortRows consecutive rows, one thread per
 // row: their bucket range (contiguous) is staged in LDS when it fits, each
 // thread sorts its row there, and the range is written back, so the sort's
 // dependent accesses are LDS round trips; a larger range is sorted in place
-// in global memory.
+// in global memory.  In a staged range, rows of more than sqrt(8 n2) atoms are
+// sorted by a wave each, by counting their bins: one lane's insertion sort
+// takes the square of the length in dependent round trips, the count a fixed
+// walk over the n2 bins.  64 molecules in 4 slices of 25 A (about 100
+// hydrogens a row, most rows empty): 382 -> 173 us.  Counting from 24 atoms on, and
+// for ranges that don't fit, measured 314 us instead of 72 for a dense 2048^2
+// slab, whose threads all have rows of one length.
+// Dynamic LDS: one count plane (n2 16-bit counts, two to a word) per counting
+// wave (sort_waves: 4, or 2 at 4096 bins, which keeps a block below 64 KB).
 constexpr int kSortRows = 256;
 constexpr uint32_t kSortLds = 16384;
-__global__ __launch_bounds__(kSortRows) void k_csr_sort_rows(int64_t n_rows,
+inline __host__ __device__ int sort_waves(int n2) { return n2 > 2048 ? 2 : kSortRows / 64; }
+__global__ __launch_bounds__(kSortRows) void k_csr_sort_rows(int64_t n_rows, int n2,
                                                              const uint32_t* __restrict__ row_start,
                                                              uint16_t* __restrict__ bucket) {
     __shared__ uint16_t lds[kSortLds];
+    __shared__ uint32_t n_long;
+    __shared__ uint2 longs[kSortRows];   // (begin, end) of the longer rows
+    extern __shared__ uint32_t sort_counts[];
     const int64_t r0 = (int64_t)blockIdx.x * kSortRows;
     const int64_t r1 = r0 + kSortRows < n_rows ? r0 + kSortRows : n_rows;
     const int64_t r = r0 + threadIdx.x;
@@ -156,10 +175,50 @@ __global__ __launch_bounds__(kSortRows) void k_csr_sort_rows(int64_t n_rows,
         if (len >= 2) sort_row(bucket + beg, len);
         return;
     }
+    if (threadIdx.x == 0) n_long = 0u;
     for (uint32_t i = threadIdx.x; i < hi - lo; i += kSortRows) lds[i] = bucket[lo + i];
     __syncthreads();
-    if (len >= 2) sort_row(lds + (beg - lo), len);
+    if (len * len > 8u * (uint32_t)n2)
+        longs[atomicAdd(&n_long, 1u)] = make_uint2(beg - lo, beg - lo + len);
+    else if (len >= 2)
+        sort_row(lds + (beg - lo), len);
     __syncthreads();
+    const int n = (int)n_long;
+    if (n > 0) {   // block-uniform
+        const int lane = threadIdx.x & 63, waves = sort_waves(n2);
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int words = n2 / 2, per = (words + 63) / 64;   // count words of a lane
+        uint32_t* cnt = sort_counts + wave * words;          // of waves below `waves`
+        for (int q = wave; wave < waves && q < n; q += waves) {
+            const uint2 row = longs[q];
+            for (int i = lane; i < words; i += 64) cnt[i] = 0u;
+            wave_lds_order();
+            for (uint32_t k = row.x + (uint32_t)lane; k < row.y; k += 64u) {
+                const uint32_t y = lds[k];
+                atomicAdd(&cnt[y >> 1], 1u << (16u * (y & 1u)));
+            }
+            wave_lds_order();
+            const int i0 = lane * per, i1 = i0 + per < words ? i0 + per : words;
+            uint32_t sum = 0u;
+            for (int i = i0; i < i1; ++i) sum += (cnt[i] & 0xffffu) + (cnt[i] >> 16);
+            uint32_t pos = sum;   // inclusive prefix over the wave's lanes
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t o = __shfl_up(pos, d);
+                if (lane >= d) pos += o;
+            }
+            pos += row.x - sum;
+            if (sum > 0u) {
+                for (int i = i0; i < i1; ++i) {
+                    const uint32_t c = cnt[i];
+                    for (uint32_t k = c & 0xffffu; k > 0u; --k) lds[pos++] = (uint16_t)(2 * i);
+                    for (uint32_t k = c >> 16; k > 0u; --k) lds[pos++] = (uint16_t)(2 * i + 1);
+                }
+            }
+            wave_lds_order();
+        }
+        __syncthreads();
+    }
     for (uint32_t i = threadIdx.x; i < hi - lo; i += kSortRows) bucket[lo + i] = lds[i];
 }
 

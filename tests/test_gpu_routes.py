@@ -184,3 +184,24 @@ def test_water_potentials_equal_dense_ones(hip, n1, n2, slices, elems, count):
         ref = builder.backend.make_slices(hist, bool(band))
         assert float((v[b] - ref).norm() / ref.norm()) < 1e-5, b
     assert torch.isfinite(image).all()
+
+
+# Row sums run over the atoms in a fixed order: the bits don't depend on the
+# order the atoms come in.  Rows sorted by a thread and by a wave (on both sides
+# of sqrt(8 n) atoms), ranges up to the sorting kernel's LDS (16384 atoms) and
+# beyond; boxes of 8 to 2048 bins.
+@pytest.mark.parametrize("n,per_row", [(64, [3] * 40), (64, [22, 23, 700] * 9), (8, [8, 9, 90, 2]),
+                                       (64, [9000, 1, 0, 7000, 380, 2, 1]), (64, [17000, 3, 1, 30]),
+                                       (512, [64, 24, 65, 0, 63] * 9), (2048, [300, 129, 26])])
+def test_image_does_not_depend_on_the_atoms_order(hip, n, per_row):
+    rng = np.random.default_rng(sum(per_row))
+    x = np.concatenate([np.full(c, k - len(per_row) // 2 + 0.5) for k, c in enumerate(per_row)])
+    xyz = np.stack([np.zeros_like(x), x, rng.uniform(-0.47 * n, 0.47 * n, len(x))],
+                   1).astype(np.float32)
+    zs = np.full(len(x), 6)
+    pipe = BatchPipe(_tem(), 1.0, 2.0, n, 2, [6, 8])
+    images = []
+    for order in (np.arange(len(x)), rng.permutation(len(x))):
+        mol = emsim_amd.atoms.AtomList(zs[order], xyz[order])
+        images.append(pipe.run(pipe.upload([pipe.prepare(mol)]))[0])
+    assert torch.isfinite(images[0]).all() and torch.equal(images[0], images[1])
