@@ -288,7 +288,17 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[EPT], float* __restric
         const int base = L::at(t);
 #pragma unroll
         for (int m = 0; m < EPT; ++m) v[m] = make_float2(re[base + L::at(m * S)], im[base + L::at(m * S)]);
-        if constexpr (SYNC2) __syncthreads();
+        if constexpr (SYNC2) {
+            // Transforms of several waves: the values are in registers here.  A
+            // caller that uses the last pass's results in a branch only (its
+            // stores) otherwise has the reads sunk into that branch, past the
+            // barrier, where the next row's writes race with them.
+            if constexpr (S > 64) {
+#pragma unroll
+                for (int m = 0; m < EPT; ++m) asm volatile("" : : "v"(v[m].x), "v"(v[m].y));
+            }
+            __syncthreads();
+        }
     }
 }
 

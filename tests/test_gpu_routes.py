@@ -205,3 +205,22 @@ def test_image_does_not_depend_on_the_atoms_order(hip, n, per_row):
         mol = emsim_amd.atoms.AtomList(zs[order], xyz[order])
         images.append(pipe.run(pipe.upload([pipe.prepare(mol)]))[0])
     assert torch.isfinite(images[0]).all() and torch.equal(images[0], images[1])
+
+
+# Rows of 1024 points and more are transformed by several waves, and a block runs
+# several rows: a row's last LDS reads come before the next row's writes.  The
+# same inputs give the same bits, and the image is the squared wave.
+@pytest.mark.parametrize("n1,n2,batch", [(512, 1024, 8), (2048, 2048, 1), (4096, 4096, 1),
+                                         (64, 4096, 40)])
+def test_long_rows_are_reproducible(hip, n1, n2, batch):
+    prop = WavePropagator(n1, n2, 1.0, 1.0, 200.0)
+    gen = torch.Generator(device="cuda").manual_seed(n1 + n2)
+    psi = torch.view_as_complex(torch.randn((batch, n1, n2, 2), generator=gen, device="cuda"))
+    wave = prop.lens_propagate(psi, 1.3, 700.0, 10e-3)
+    image = prop.lens_intensity(psi, 1.3, 700.0, 10e-3)
+    for _ in range(4):
+        assert torch.equal(prop.lens_propagate(psi, 1.3, 700.0, 10e-3), wave)
+        assert torch.equal(prop.lens_intensity(psi, 1.3, 700.0, 10e-3), image)
+    # float32 against float32 of the same wave: a few roundings of the square
+    square = wave.abs().double() ** 2
+    assert float((image.double() - square).norm() / square.norm()) < 1e-6
