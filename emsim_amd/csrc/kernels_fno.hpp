@@ -2,8 +2,9 @@
 // (lifting, spectral layers, projection) on channels-last activations, and
 // its backward pass and optimiser.
 //
-// Every dense contraction is one call of k_gemm: a batched, strided GEMM
-// on bf16 MFMA (v_mfma_f32_32x32x16_bf16) with float32 accumulation.
+// Every dense contraction that no fused row or x-transform kernel below takes is
+// one call of k_gemm: a batched, strided GEMM on bf16 MFMA
+// (v_mfma_f32_32x32x16_bf16) with float32 accumulation.
 // Operands are float32 or bf16 in memory and are rounded to bf16 (nearest
 // even) when staged in LDS; an optional second operand pair extends the
 // sum over k (used to fuse the pointwise channel mix with the inverse
