@@ -289,14 +289,16 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[EPT], float* __restric
 #pragma unroll
         for (int m = 0; m < EPT; ++m) v[m] = make_float2(re[base + L::at(m * S)], im[base + L::at(m * S)]);
         if constexpr (SYNC2) {
-            // Transforms of several waves: the values are in registers here.  A
-            // caller that uses the last pass's results in a branch only (its
-            // stores) otherwise has the reads sunk into that branch, past the
-            // barrier, where the next row's writes race with them.
-            if constexpr (S > 64) {
+            // The values are in registers here.  A caller that uses the last
+            // pass's results under a block-uniform condition only (its stores)
+            // otherwise has the reads sunk into that branch, past the barrier,
+            // where another wave's writes for the block's next transform race
+            // with them.  Whether a transform spans waves is the caller's
+            // choice of t (several columns side by side spread even a short
+            // one over the block), so every pass with this barrier is pinned;
+            // it adds no instructions.
 #pragma unroll
-                for (int m = 0; m < EPT; ++m) asm volatile("" : : "v"(v[m].x), "v"(v[m].y));
-            }
+            for (int m = 0; m < EPT; ++m) asm volatile("" : : "v"(v[m].x), "v"(v[m].y));
             __syncthreads();
         }
     }
