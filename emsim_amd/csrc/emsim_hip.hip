@@ -781,14 +781,14 @@ int launch_chirp_spectrum(float2* X, const float* sf, int n_elems, int sc, int H
 }
 
 template <int M>
-int launch_chirp_c2r(const float2* X, float* out, int64_t rows, int ldh, float clip_lo,
+int launch_chirp_c2r(const float2* X, float* out, int sc, int n1, int ldh, float clip_lo,
                      const ChirpTab& row, const float2* tw, hipStream_t s) {
     static int resident_cache[64];
     int rpb;
     dim3 grid;
-    row_grid<M>((rows + 1) / 2, rpb, grid,
+    row_grid<M>((int64_t)sc * ((n1 + 1) / 2), rpb, grid,
                 resident_blocks(k_chirp_c2r<M>, RowCfg<M>::BLOCK, resident_cache));
-    EMSIM_LAUNCH(M, (k_chirp_c2r<M>), grid, dim3(RowCfg<M>::BLOCK), 0, s, X, out, rows, ldh, rpb,
+    EMSIM_LAUNCH(M, (k_chirp_c2r<M>), grid, dim3(RowCfg<M>::BLOCK), 0, s, X, out, sc, n1, ldh, rpb,
                  clip_lo, row, tw);
     return EMSIM_HIP_OK;
 }
@@ -829,9 +829,9 @@ int chirp_spectrum(int M, float2* X, const float* sf, int n_elems, int sc, int H
     EMSIM_CHIRP_DISPATCH(M, launch_chirp_spectrum, X, sf, n_elems, sc, H, ldh, n2, bandlimit,
                          band_r2, inv_npix, col, tw, s);
 }
-int chirp_c2r(int M, const float2* X, float* out, int64_t rows, int ldh, float clip_lo,
+int chirp_c2r(int M, const float2* X, float* out, int sc, int n1, int ldh, float clip_lo,
               const ChirpTab& row, const float2* tw, hipStream_t s) {
-    EMSIM_CHIRP_DISPATCH(M, launch_chirp_c2r, X, out, rows, ldh, clip_lo, row, tw, s);
+    EMSIM_CHIRP_DISPATCH(M, launch_chirp_c2r, X, out, sc, n1, ldh, clip_lo, row, tw, s);
 }
 
 // Row-pass arguments of a batch of waves (V: one slice's potentials, or null).
@@ -1174,8 +1174,8 @@ extern "C" int emsim_hip_make_slices(const emsim_hip_slice_builder* b, const flo
                                 symmetric_bandlimit ? 1 : 0, r * r, inv_npix, b->p1.tab(), b->tw,
                                 s);
             if (rc) return rc;
-            rc = chirp_c2r(b->p2.M, X, out + (int64_t)s0 * b->n1 * b->n2, (int64_t)sc * b->n1, ldh,
-                           1e-13f, b->p2.tab(), b->tw, s);
+            rc = chirp_c2r(b->p2.M, X, out + (int64_t)s0 * b->n1 * b->n2, sc, b->n1, ldh, 1e-13f,
+                           b->p2.tab(), b->tw, s);
             if (rc) return rc;
         }
         return EMSIM_HIP_OK;

@@ -470,11 +470,12 @@ __global__ __launch_bounds__((ChirpColCfg<M, NARROW>::BLOCK)) void k_chirp_spect
     }
 }
 
-// rows: sc * n1 half rows in (ldh apart), pairs (2q, 2q + 1) over all of them;
-// real rows out, n apart.
+// planes of n1 half rows in (ldh apart), pairs (2q, 2q + 1) within each plane, so
+// that no slice's values (an infinity's NaN, a rounding) reach another one's rows
+// where n1 is odd; real rows out, n apart.
 template <int M>
 __global__ __launch_bounds__(RowCfg<M>::BLOCK) void k_chirp_c2r(
-    const float2* __restrict__ X, float* __restrict__ out, int64_t rows, int ldh, int rpb,
+    const float2* __restrict__ X, float* __restrict__ out, int planes, int n1, int ldh, int rpb,
     float clip_lo, ChirpTab row, const float2* __restrict__ tw) {
     using Cfg = RowCfg<M>;
     constexpr int EPT = Cfg::EPT, HALF = EPT / 2, T = Cfg::T;
@@ -484,8 +485,8 @@ __global__ __launch_bounds__(RowCfg<M>::BLOCK) void k_chirp_c2r(
     const int t = threadIdx.x % T;
     float* re = lds_re + gi * Cfg::WORDS;
     float* im = lds_im + gi * Cfg::WORDS;
-    const int n = row.n;
-    const int64_t pairs = (rows + 1) / 2;
+    const int n = row.n, ppp = (n1 + 1) / 2;   // pairs per plane
+    const int64_t pairs = (int64_t)planes * ppp;
     float2 b[EPT], c[HALF];
     chirp_load_b<M, EPT>(row.b, t, b);
 #pragma unroll
@@ -495,10 +496,18 @@ __global__ __launch_bounds__(RowCfg<M>::BLOCK) void k_chirp_c2r(
     struct Regs {
         float2 a[HALF], b[HALF];
     } cur, nxt;
+    // the pair's first row (of all planes'), and whether it has a second one
+    auto locate = [&](int64_t p0, bool& two) __attribute__((always_inline)) {
+        const int64_t p = p0 < pairs ? p0 : pairs - 1;
+        const int64_t plane = p / ppp;
+        const int x = 2 * (int)(p - plane * ppp);
+        two = x + 1 < n1;
+        return plane * n1 + x;
+    };
     auto load = [&](int64_t p0, Regs& g) __attribute__((always_inline)) {
-        const int64_t ra = 2 * (p0 < pairs ? p0 : pairs - 1);
-        const float2* ia = X + ra * ldh;
-        const float2* ib = ra + 1 < rows ? ia + ldh : ia;
+        bool two;
+        const float2* ia = X + locate(p0, two) * ldh;
+        const float2* ib = two ? ia + ldh : ia;
 #pragma unroll
         for (int m = 0; m < HALF; ++m) {
             const int k = t + m * T, kc = k < n ? k : n - 1;
@@ -510,9 +519,10 @@ __global__ __launch_bounds__(RowCfg<M>::BLOCK) void k_chirp_c2r(
     const int64_t first = (int64_t)blockIdx.x * rpb * Cfg::G + gi;
     load(first, cur);
     for (int r = 0; r < rpb; ++r) {
-        const int64_t p = first + (int64_t)r * Cfg::G, ra = 2 * p;
+        const int64_t p = first + (int64_t)r * Cfg::G;
         if (r + 1 < rpb) load(p + Cfg::G, nxt);
-        const bool two = ra + 1 < rows;
+        bool two;
+        const int64_t ra = locate(p, two);
         float2 v[EPT];
 #pragma unroll
         for (int m = 0; m < HALF; ++m) {

@@ -68,3 +68,24 @@ def test_slices(hip, n, slices, elems):
         got = builder.make_multi_slices(hist, limit).cpu().numpy()
         ref = orc.make_multi_slices_f64(hist, sf, limit)
         assert orc.rel_l2(got, ref) < TOL
+
+
+@pytest.mark.parametrize("n1,n2,slices", [(75, 75, 6), (33, 64, 5), (9, 100, 7)])
+def test_slices_do_not_mix(hip, n1, n2, slices):
+    """Each slice of a grid of odd n1 comes from its own counts alone: the same
+    bits with one slice or several to a launch, and with infinite counts in the
+    slice before it."""
+    elems = [1, 6]
+    rng = np.random.default_rng(n1)
+    hist = rng.poisson(0.2, (len(elems), slices, n1, n2)).astype(np.float32)
+    limit = n1 == n2
+    builder = MultiSlicesBuilder(elems, slices, n1, n2, 2.0, 1.0, 1.0)
+    one = MultiSlicesBuilder(elems, 1, n1, n2, 2.0, 1.0, 1.0)
+    got = builder.make_multi_slices(hist, limit)
+    for s in range(slices):
+        alone = one.make_multi_slices(np.ascontiguousarray(hist[:, s:s + 1]), limit)
+        assert torch.equal(alone[0], got[s]), s
+    hist[1, 2, n1 // 2, 3] = np.inf
+    again = builder.make_multi_slices(hist, limit)
+    for s in range(slices):
+        assert s == 2 or torch.equal(again[s], got[s]), s
