@@ -1735,16 +1735,20 @@ bool fused_split(const emsim_hip_slice_builder* b, int batch) {
 // kMinChunk: their planes spill to HBM, but one launch of many rounds has one
 // tail instead of one per slice (64 of 512^2 x 100: 18.53 ms at one slice,
 // 18.12 ms at seven; 64 / 128 / 192 / 256 MB with no minimum measured 6,145 /
-// 5,478 / 5,352 / 5,424 us for 32 of 512^2 x 50).
+// 5,478 / 5,352 / 5,424 us for 32 of 512^2 x 50).  That tail matters less the
+// longer one slice's launch already is, so the minimum ends at kMaxChunkBytes
+// of planes: a batch whose single slice is as large takes one slice at a time
+// and no more workspace than that.
 constexpr int64_t kChunkBytes = (int64_t)192 << 20;
 constexpr int64_t kMinChunk = 8;
+constexpr int64_t kMaxChunkBytes = (int64_t)2 << 30;
 int fused_chunk(const emsim_hip_slice_builder* b, int batch, bool water) {
     const int64_t rows = (int64_t)batch * b->n1;
     const int64_t per = rows * (fused_ld(b) + (fused_split(b, batch) ? b->n2 : 0) +
                                 (water ? 2 * half_ld(b->H) : 0)) *
                         (int64_t)sizeof(float2);
-    const int64_t c = std::max(kChunkBytes / per, kMinChunk);
-    return (int)std::min(c, (int64_t)b->n_slices);
+    const int64_t least = std::min(kMinChunk, std::max<int64_t>(kMaxChunkBytes / per, 1));
+    return (int)std::min(std::max(kChunkBytes / per, least), (int64_t)b->n_slices);
 }
 
 struct FusedWorkspace {

@@ -185,7 +185,10 @@ int emsim_hip_intensity(const float* wave_dev, float* out_dev, int64_t n,
  * With a one-slice builder this is the weak-phase-object path of
  * emsim/pipe.py:57-64,73-77 for the whole batch: the 2-D projected potential
  * (z ignored, slice_builder_base.py:202-225), transmission, then
- * singleslice_propagate(dz = 0) -- the propagator's mask alone. */
+ * singleslice_propagate(dz = 0) -- the propagator's mask alone.
+ * The workspace holds, besides the wave and the atoms' bins, the half spectra
+ * (small batches: and the transmission functions) of several slices: as many
+ * as fit 192 MiB, at least 8 while they stay within 2 GiB, at least 1. */
 size_t emsim_hip_simulate_workspace_size(const emsim_hip_slice_builder* b, int batch,
                                          int64_t n_atoms, int mode);
 int emsim_hip_simulate(const emsim_hip_slice_builder* b, const emsim_hip_wave_propagator* w,

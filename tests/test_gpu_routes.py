@@ -224,3 +224,35 @@ def test_long_rows_are_reproducible(hip, n1, n2, batch):
     # float32 against float32 of the same wave: a few roundings of the square
     square = wave.abs().double() ** 2
     assert float((image.double() - square).norm() / square.norm()) < 1e-6
+
+
+def _workspace_bytes(n, slices, batch, water):
+    builder = MultiSlicesBuilder(ELEMS, slices, n, n, 2.0, 1.0, 1.0).backend
+    name = f"emsim_hip_simulate{'_water' if water else ''}_workspace_size"
+    return hip_ext.raw(name)(builder.h, batch, 1000, 0)
+
+
+# Planes of several slices are workspace that a batch of one slice at a time does
+# not need: 2 GiB of them at most, and none beyond the first slice where that one
+# is larger.  (The atoms' row table: 2 x 4 bytes a row, 4 per molecule, and a sum of 4
+# bytes per tile of its scan, 2048 rows.)
+@pytest.mark.parametrize("n,batch", [(256, 64), (512, 64), (2048, 16), (2048, 64), (4096, 1),
+                                     (4096, 100)])
+@pytest.mark.parametrize("water", [False, True])
+def test_workspace_of_several_slices_is_bounded(hip, n, batch, water):
+    slices = 16
+    rows = (slices - 1) * batch * len(ELEMS) * n
+    tables = 8 * rows + 4 * (rows // 2048) + 4 * (slices - 1) * batch + 4096
+    one = _workspace_bytes(n, 1, batch, water)
+    more = _workspace_bytes(n, slices, batch, water) - one - tables
+    plane = batch * n * (n // 2 + 1) * 8 * (3 if water else 1)
+    assert more <= (2 << 30) - plane or (plane > 1 << 30 and more <= 0)
+
+
+def test_image_does_not_depend_on_the_bounded_planes(hip):
+    """16 images of 2048^2: seven slices to a launch by that bound, eleven alone."""
+    pipe = BatchPipe(_tem(), 1.0, 2.0, 2048, 9, ELEMS)
+    prepared = [pipe.prepare(synth.protein_cloud(2000 + 300 * k, 70 + k)) for k in range(2)]
+    images = pipe.run(pipe.upload([prepared[k % 2] for k in range(16)]))
+    for k in range(2):
+        assert torch.equal(pipe.run(pipe.upload([prepared[k]]))[0], images[k])
