@@ -1731,24 +1731,37 @@ bool fused_split(const emsim_hip_slice_builder* b, int batch) {
 // takes as many slices at once as fit kChunkBytes of planes -- most of the
 // 256 MB cache behind the L2s, from which they are read back -- instead of
 // one part-filled round of blocks per slice (one 256^2 image, 45 slices:
-// 1,526 -> 740 us; 64 of 256^2 4,124 -> 3,440 us).  Large batches still take
-// kMinChunk: their planes spill to HBM, but one launch of many rounds has one
-// tail instead of one per slice (64 of 512^2 x 100: 18.53 ms at one slice,
-// 18.12 ms at seven; 64 / 128 / 192 / 256 MB with no minimum measured 6,145 /
-// 5,478 / 5,352 / 5,424 us for 32 of 512^2 x 50).  That tail matters less the
-// longer one slice's launch already is, so the minimum ends at kMaxChunkBytes
-// of planes: a batch whose single slice is as large takes one slice at a time
-// and no more workspace than that.
+// 1,526 -> 740 us; 64 of 256^2 4,124 -> 3,440 us; 64 / 128 / 192 / 256 MB
+// measured 6,145 / 5,478 / 5,352 / 5,424 us for 32 of 512^2 x 50).
+// Planes that don't fit come back from HBM, but one launch of many rounds has
+// one tail instead of one per slice, so larger batches take kMinChunk: 256
+// images of 512^2 x 30 26.4 ms at one slice, 25.2 at eight.  From 512 to 2048
+// rows the tail is worth it where not even two slices fit, or where blocks run
+// long because a slice has kDenseRow atoms and more per row (64 of 512^2 x 4,
+// 20 a row, at two slices 1.87 ms, four 1.83; x 8, 49 a row, 6.13 and at eight
+// 5.97).  Otherwise the planes stay in the cache: 64 of 512^2 x 100, 0.8 a row,
+// at two slices 17.35 ms, three 17.95, eight 17.65; with atoms in half those
+// slices 13.17 and 14.03; x 20, 4 a row, 4.49 and 4.55; x 8, 10 a row, 2.38 and
+// 2.39; four of 2048^2 x 40, 4 a row, at three slices 22.1, eight 22.4; x 12, 12
+// a row, 8.09 and 8.06.  256 images of 256^2 x 40 measured 9.39 at two, 9.20 at
+// eight, and one of 4096^2 x 20 13.42 and 13.12.
+// The minimum ends at kMaxChunkBytes: a batch whose single slice is as large
+// takes one slice at a time and no more workspace than that (64 of 2048^2 x 8
+// 68.7 ms, 76.1 at eight slices).
 constexpr int64_t kChunkBytes = (int64_t)192 << 20;
 constexpr int64_t kMinChunk = 8;
 constexpr int64_t kMaxChunkBytes = (int64_t)2 << 30;
-int fused_chunk(const emsim_hip_slice_builder* b, int batch, bool water) {
+constexpr int64_t kDenseRow = 12;
+int fused_chunk(const emsim_hip_slice_builder* b, int batch, int64_t n_atoms, bool water) {
     const int64_t rows = (int64_t)batch * b->n1;
     const int64_t per = rows * (fused_ld(b) + (fused_split(b, batch) ? b->n2 : 0) +
                                 (water ? 2 * half_ld(b->H) : 0)) *
                         (int64_t)sizeof(float2);
-    const int64_t least = std::min(kMinChunk, std::max<int64_t>(kMaxChunkBytes / per, 1));
-    return (int)std::min(std::max(kChunkBytes / per, least), (int64_t)b->n_slices);
+    int64_t c = std::max<int64_t>(kChunkBytes / per, 1);
+    const bool dense = n_atoms / b->n_slices >= kDenseRow * rows;
+    if (c < 2 || dense || b->n1 < 512 || b->n1 > 2048)
+        c = std::max(c, std::min(kMinChunk, kMaxChunkBytes / per));
+    return (int)std::min(c, (int64_t)b->n_slices);
 }
 
 struct FusedWorkspace {
@@ -1789,7 +1802,7 @@ struct WaterFill {
 FusedWorkspace fused_layout(const emsim_hip_slice_builder* b, int batch, int64_t n_atoms,
                             bool own_wave, char* base, bool water = false, bool raw = false) {
     FusedWorkspace w;
-    w.chunk = fused_chunk(b, batch, water);
+    w.chunk = fused_chunk(b, batch, n_atoms, water);
     w.n_rows = (int64_t)batch * b->n_slices * b->n_elems * b->n1;
     const int64_t n_scan = w.n_rows + 1;
     const int64_t n_blocks = ceil_div(n_scan, kScanTile);

@@ -188,7 +188,7 @@ int emsim_hip_intensity(const float* wave_dev, float* out_dev, int64_t n,
  * singleslice_propagate(dz = 0) -- the propagator's mask alone.
  * The workspace holds, besides the wave and the atoms' bins, the half spectra
  * (small batches: and the transmission functions) of several slices: as many
- * as fit 192 MiB, at least 8 while they stay within 2 GiB, at least 1. */
+ * as fit 192 MiB, up to 8 beyond that within 2 GiB, at least 1. */
 size_t emsim_hip_simulate_workspace_size(const emsim_hip_slice_builder* b, int batch,
                                          int64_t n_atoms, int mode);
 int emsim_hip_simulate(const emsim_hip_slice_builder* b, const emsim_hip_wave_propagator* w,

@@ -256,3 +256,14 @@ def test_image_does_not_depend_on_the_bounded_planes(hip):
     images = pipe.run(pipe.upload([prepared[k % 2] for k in range(16)]))
     for k in range(2):
         assert torch.equal(pipe.run(pipe.upload([prepared[k]]))[0], images[k])
+
+
+# 512 to 2048 rows: where two slices' planes fit the cache behind the L2s (192 MiB
+# of them), a launch takes no more than fit it.
+@pytest.mark.parametrize("n,batch", [(512, 16), (512, 64), (1024, 16), (2048, 2), (2048, 4)])
+def test_planes_that_fit_the_cache_stay_in_it(hip, n, batch):
+    slices = 16
+    rows = (slices - 1) * batch * len(ELEMS) * n
+    tables = 8 * rows + 4 * (rows // 2048) + 4 * (slices - 1) * batch + 4096
+    more = _workspace_bytes(n, slices, batch, False) - _workspace_bytes(n, 1, batch, False)
+    assert more - tables <= (192 << 20) - batch * n * (n // 2 + 1) * 8
