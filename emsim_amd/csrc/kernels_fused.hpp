@@ -1044,7 +1044,7 @@ struct OpSlicePassA {
     // the run, and this pass never stores into them, so no load needs a
     // branch.  From 512 columns on all the zeros are read from one dead column,
     // whose line stays in the L1, which takes a third of the wave's reads off
-    // the caches behind it (64 of 512^2 x 100 slices 17.76 -> 17.48 ms); at
+    // the caches behind it (64 of 512^2 x 100 slices 18.45 -> 17.50 ms); at
     // 256 columns the per-element offsets cost more (64 of 256^2 x 45 slices
     // 3,311 -> 3,340 us), so they are loaded as they are.
     static constexpr bool kOneZero = N >= 512;

@@ -272,7 +272,10 @@ struct OpTransmit {
 #pragma unroll
         for (int m = 0; m < EPT; ++m) {
             // the dead columns' zeros all from one of them: its line stays in
-            // the L1 while the others' would come from beyond the L2
+            // the L1 while the others' would come from beyond the L2 (16 waves
+            // of 512^2 through 50 slices of their own 1,931 -> 1,864 us; 40
+            // shared slices: 16 of 256^2 796 -> 785, 64 of 128^2 769 -> 763,
+            // but 16 of 512^2, with the caches to themselves, 1,390 -> 1,410)
             const int k = t + m * T;
             const int kw = !FIRST && dead(k) ? dead_lo : k;
             r.v[m] = ok ? src[kw] : make_float2(0.f, 0.f);
