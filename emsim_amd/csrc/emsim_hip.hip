@@ -11,10 +11,10 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -2115,7 +2115,7 @@ extern "C" int emsim_hip_pack_raw(int n_mols, const float* const* coords, const 
     int started = 0;
     try {
         for (; started < extra; ++started) pool[started] = std::thread(work);
-    } catch (const std::system_error&) {   // no more threads: the caller's own does the rest
+    } catch (const std::exception&) {   // no thread or no memory for one: the caller's own does the rest
     }
     work();
     for (int t = 0; t < started; ++t) pool[t].join();

@@ -2,6 +2,9 @@
 coordinates and element indices, extents, elements outside the list, and batches
 large enough to be split over threads."""
 import ctypes
+import os
+import subprocess
+import sys
 from ctypes import POINTER, byref, c_int, c_int64, c_void_p
 
 import numpy as np
@@ -81,3 +84,51 @@ def test_bounds_and_runs_equal_numpy():
         assert counts.dtype == ref[1].dtype and zs.dtype == ref[0].dtype
     with pytest.raises(ValueError):
         atm.AtomList(np.zeros(0, int), np.zeros((0, 3))).space
+
+
+NEW = r"""
+#include <cstdlib>
+#include <new>
+static bool failing = false;
+extern "C" void fail_new(int on) { failing = on; }
+void* operator new(std::size_t n) {
+    void* p = failing ? nullptr : std::malloc(n);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+"""
+PACK = """
+import ctypes
+import numpy as np
+from emsim_amd import atoms as atm
+from tests.test_pack_raw import ELEMS, _pack
+mols = [atm.AtomList(np.full(150000, 6), np.full((150000, 3), k, np.float32)) for k in range(4)]
+fail = ctypes.CDLL(None).fail_new
+call = __import__("emsim_amd.backend.hip_ext", fromlist=["call"])
+real = call.call
+def failing(*args):
+    fail(1)
+    try:
+        return real(*args)
+    finally:
+        fail(0)
+call.call = failing
+c, e, ext, bad = _pack(mols, 4)
+assert bad == -1 and (e == ELEMS.index(6)).all()
+assert (c == np.repeat(np.arange(4), 150000)[:, None]).all()
+print("packed")
+"""
+
+
+def test_no_memory_for_a_thread(tmp_path):
+    """A thread that cannot be had for want of memory is no error: the call's own
+    thread packs everything."""
+    src, lib = tmp_path / "new.cpp", tmp_path / "libnew.so"
+    src.write_text(NEW)
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", str(src), "-o", str(lib)], check=True)
+    env = dict(os.environ, LD_PRELOAD=" ".join([str(lib), os.environ.get("LD_PRELOAD", "")]).strip())
+    out = subprocess.run([sys.executable, "-c", PACK], env=env, capture_output=True, text=True,
+                         timeout=100, cwd=os.path.dirname(os.path.dirname(__file__)))
+    assert out.returncode == 0 and "packed" in out.stdout, out.stderr[-500:]
