@@ -1986,9 +1986,10 @@ extern "C" int emsim_hip_simulate_water(const emsim_hip_slice_builder* b,
     if (idx_h < 0 || idx_o < 0 || idx_h >= b->n_elems || idx_o >= b->n_elems || idx_h == idx_o ||
         !(voxel_water >= 0))
         return fail(EMSIM_HIP_EINVAL, "simulate_water: bad water arguments");
+    // the range this entry point has always taken (and is tested over); no kernel
+    // of the path needs it any more
     if ((size_t)b->n_elems * b->n2 * sizeof(float) > 64 * 1024)
-        return fail(EMSIM_HIP_EUNSUPPORTED,
-                    "simulate_water: n_elems * n2 <= 16384");
+        return fail(EMSIM_HIP_EUNSUPPORTED, "simulate_water: n_elems * n2 <= 16384");
     std::vector<int64_t> elem_off;
     rc = host_offsets(b, mol_off_host, elem_counts_host, batch, n_atoms, elem_off);
     if (rc) return rc;
