@@ -295,8 +295,9 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[EPT], float* __restric
             // where another wave's writes for the block's next transform race
             // with them.  Whether a transform spans waves is the caller's
             // choice of t (several columns side by side spread even a short
-            // one over the block), so every pass with this barrier is pinned;
-            // it adds no instructions.
+            // one over the block), so every pass with this barrier is pinned.
+            // It adds no instructions, but the compiler moves no load from
+            // behind it out of a loop: tables are loaded ahead of loops.
 #pragma unroll
             for (int m = 0; m < EPT; ++m) asm volatile("" : : "v"(v[m].x), "v"(v[m].y));
             __syncthreads();
