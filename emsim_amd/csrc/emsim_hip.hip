@@ -1745,6 +1745,10 @@ bool fused_split(const emsim_hip_slice_builder* b, int batch) {
 // 2.39; four of 2048^2 x 40, 4 a row, at three slices 22.1, eight 22.4; x 12, 12
 // a row, 8.09 and 8.06.  256 images of 256^2 x 40 measured 9.39 at two, 9.20 at
 // eight, and one of 4096^2 x 20 13.42 and 13.12.
+// A run of up to four slices whose planes all together take at most half as much
+// again goes in one launch, which mostly still finds them in the cache (64 of
+// 512^2 x 4, 11 a row, 1.63 ms in two launches, 1.59 in one; four of 2048^2 x 3
+// 1.78 and 1.75).
 // The minimum ends at kMaxChunkBytes: a batch whose single slice is as large
 // takes one slice at a time and no more workspace than that (64 of 2048^2 x 8
 // 68.7 ms, 76.1 at eight slices).
@@ -1757,6 +1761,7 @@ int fused_chunk(const emsim_hip_slice_builder* b, int batch, int64_t n_atoms, bo
     const int64_t per = rows * (fused_ld(b) + (fused_split(b, batch) ? b->n2 : 0) +
                                 (water ? 2 * half_ld(b->H) : 0)) *
                         (int64_t)sizeof(float2);
+    if (b->n_slices <= 4 && b->n_slices * per <= kChunkBytes / 2 * 3) return b->n_slices;
     int64_t c = std::max<int64_t>(kChunkBytes / per, 1);
     const bool dense = n_atoms / b->n_slices >= kDenseRow * rows;
     if (c < 2 || dense || b->n1 < 512 || b->n1 > 2048)
